@@ -37,6 +37,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <type_traits>
+#include <atomic>
 #include "../../include/jkhip.h"
 
 #define PI_FAC          34.98683665524972497    // 2 pi^(5/2)
@@ -193,6 +194,17 @@ __device__ __forceinline__ void select_replica(JKBuildArgs &a)
 // LDS accumulation: workgroup scope, so that it cannot be merged with the
 // device-scope HBM atomics of a sibling branch into one generic atomic
 __device__ __forceinline__ void lds_add(double *p, double v)
+{
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// A double in LDS by its own address space: where a value comes from LDS in one
+// branch and from HBM in the other, generic pointers let the compiler merge the
+// two loads into a flat one, which is slower than either and completes only
+// behind the wavefront's outstanding atomics.
+typedef __attribute__((address_space(3))) double lds_double;
+
+__device__ __forceinline__ void lds_add(lds_double *p, double v)
 {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -688,31 +700,81 @@ struct WorkItem { int pij, kl0, kl1, k_ao0, k_nao, l_ao0, l_nao; };
 #define KR_DROWS        4       // density rows staged too
 #define KR_WIN          8       // work items = ij pairs x kl column windows
 
-// Workgroups are dispatched round-robin over the XCDs (each with its own
-// L2): block b runs on XCD b % NXCD.  With XCD_SWIZZLE the blocks of one XCD
-// take a contiguous range of work items (same ij pairs, neighbouring kl
-// chunks), a bijection of [0, gridDim.x) for any grid size.  It is off: the
-// ij pair lists are sorted by descending Schwarz bound, so contiguous ranges
-// hand one XCD the heaviest work items (32-water def2-TZVP build: 1056 ms
-// with it, 652 ms with the round-robin order).
-#ifndef XCD_SWIZZLE
-#define XCD_SWIZZLE 0
-#endif
-#define NXCD 8
-__device__ __forceinline__ int work_index()
+// A batched launch runs up to JK_BATCH tasks of one angular class: workgroup b
+// belongs to the last task t with block0[t] <= b.  The class kernels of a
+// small molecule are latency bound (one wavefront of quartets, a serial loop
+// over the primitives), so what a build costs is the number of launches in a
+// row: def2-SVP has 266 tasks but 21 angular classes, def2-TZVP 750 and 55.
+// Building them class by class took one water molecule (def2-SVP) from 3.65 to
+// 1.23 ms, 8 from 8.46 to 2.90 ms and 48 (def2-TZVP) from 1048 to 1020 ms.
+// JK_BATCH descriptors and the shared arguments fill the 4 KB of kernel
+// arguments, which reach the kernel through scalar loads; no descriptor is
+// copied to device memory.
+#define JK_BATCH 31
+struct TaskDesc {
+    const uint32_t *pairs_ij, *pairs_kl;
+    const float *q_ij, *q_kl;
+    const double *pdata_ij, *pdata_kl;
+    const int32_t *win;             // kl column windows (KR_WIN)
+    int npairs_ij, npairs_kl;
+    uint32_t prims_ij, prims_kl;    // iprim | jprim << 16, kprim | lprim << 16
+    int k_ao0, k_nao, l_ao0, l_nao;
+    int kl_chunk;                   // candidates per work item (not KR_WIN)
+    int use_lds;                    // KR_* bits
+    int counter;                    // element of the per-task counters
+    uint32_t ls_swap;               // li, lj, lk, ll, 4 bits each, and swap_ijkl << 16
+};
+struct TaskBatch {
+    int n, pad;
+    int block0[JK_BATCH + 1];       // first workgroup of each task, INT_MAX past n
+    TaskDesc t[JK_BATCH];
+};
+static_assert(sizeof(JKBuildArgs) + sizeof(TaskBatch) + 64 <= 4096, "kernel arguments above 4 KB");
+
+// A descriptor's pointer as one to global memory: the compiler takes that for
+// granted for pointers among the kernel arguments, but not for those of a
+// descriptor at a runtime index, whose accesses would become flat ones (no
+// scalar base, 12 more registers and the LDS counter: (dp|ss) 18.4 -> 26.6 ms,
+// (fp|dp) 34 -> 52 ms of the 48-water def2-TZVP build).
+template <typename T>
+__device__ __forceinline__ T *as_global(T *p)
 {
-    const int b = blockIdx.x;
-    if (!XCD_SWIZZLE) return b;
-    const int n = gridDim.x;
-    const int x = b % NXCD, per = n / NXCD, rem = n % NXCD;
-    return x * per + (x < rem ? x : rem) + b / NXCD;
+    return (T *)(__attribute__((address_space(1))) T *)p;
 }
 
-__device__ __forceinline__ WorkItem work_item(int npairs_kl, int kl_chunk)
+// The task of this workgroup: its fields into the launch's arguments;
+// returns the workgroup's index within the task.
+__device__ __forceinline__ int select_task(JKBuildArgs &a, const TaskBatch &b, int &kl_chunk,
+                                           int &use_lds)
+{
+    const int blk = blockIdx.x;
+    int t = 0;
+#pragma unroll
+    for (int n = 1; n < JK_BATCH; ++n) t = blk >= b.block0[n] ? n : t;
+    const TaskDesc &d = b.t[t];
+    a.li = d.ls_swap & 15; a.lj = d.ls_swap >> 4 & 15;
+    a.lk = d.ls_swap >> 8 & 15; a.ll = d.ls_swap >> 12 & 15;
+    a.swap_ijkl = d.ls_swap >> 16;
+    a.pairs_ij = as_global(d.pairs_ij); a.pairs_kl = as_global(d.pairs_kl);
+    a.q_ij = as_global(d.q_ij); a.q_kl = as_global(d.q_kl);
+    a.pdata_ij = as_global(d.pdata_ij); a.pdata_kl = as_global(d.pdata_kl);
+    a.kl_win[0].win = as_global(d.win);
+    a.npairs_ij = d.npairs_ij; a.npairs_kl = d.npairs_kl;
+    a.iprim = d.prims_ij & 0xffff; a.jprim = d.prims_ij >> 16;
+    a.kprim = d.prims_kl & 0xffff; a.lprim = d.prims_kl >> 16;
+    a.k_ao0 = d.k_ao0; a.k_nao = d.k_nao; a.l_ao0 = d.l_ao0; a.l_nao = d.l_nao;
+    if (a.n_quartets) a.n_quartets += d.counter;
+    if (a.n_quartets_fp32) a.n_quartets_fp32 += d.counter;
+    if (a.quartet_hash) a.quartet_hash += d.counter;
+    kl_chunk = d.kl_chunk;
+    use_lds = d.use_lds;
+    return blk - b.block0[t];
+}
+
+__device__ __forceinline__ WorkItem work_item(int idx, int npairs_kl, int kl_chunk)
 {
     int nchunks = (npairs_kl + kl_chunk - 1) / kl_chunk;
     WorkItem w;
-    const int idx = work_index();
     w.pij = idx / nchunks;
     int ch = idx - w.pij * nchunks;
     w.kl0 = ch * kl_chunk;
@@ -724,10 +786,9 @@ __device__ __forceinline__ WorkItem work_item(int npairs_kl, int kl_chunk)
 // work items over the kl column windows of kl_win[0] (window major, ij pair
 // minor; the launcher puts the team kernels' set there); the K-row columns
 // are the window's
-__device__ __forceinline__ WorkItem work_item_win(const JKBuildArgs &a)
+__device__ __forceinline__ WorkItem work_item_win(const JKBuildArgs &a, int idx)
 {
     WorkItem w;
-    const int idx = work_index();
     const int win = idx / a.npairs_ij;
     w.pij = idx - win * a.npairs_ij;
     const int32_t *d = a.kl_win[0].win + 6 * win;
@@ -736,12 +797,13 @@ __device__ __forceinline__ WorkItem work_item_win(const JKBuildArgs &a)
     return w;
 }
 
-// work item of a per-lane or team launch: kl chunks over the whole groups,
+// work item idx of a per-lane or team task: kl chunks over the whole groups,
 // or the kl column windows
-__device__ __forceinline__ WorkItem work_item(const JKBuildArgs &a, int kl_chunk, int use_lds)
+__device__ __forceinline__ WorkItem work_item(const JKBuildArgs &a, int idx, int kl_chunk,
+                                              int use_lds)
 {
-    if (use_lds & KR_WIN) return work_item_win(a);
-    WorkItem w = work_item(a.npairs_kl, kl_chunk);
+    if (use_lds & KR_WIN) return work_item_win(a, idx);
+    WorkItem w = work_item(idx, a.npairs_kl, kl_chunk);
     w.k_ao0 = a.k_ao0; w.k_nao = a.k_nao; w.l_ao0 = a.l_ao0; w.l_nao = a.l_nao;
     return w;
 }
@@ -752,11 +814,11 @@ __device__ __forceinline__ WorkItem work_item(const JKBuildArgs &a, int kl_chunk
 // The same row layout also holds, after the K rows, a copy of the density
 // rows i and j over the k and l group columns (dstaged), from which the
 // per-lane digestion reads D_ik, D_il, D_jk and D_jl.
-// p and d always point into the LDS array (so that every access compiles
-// to an LDS instruction); `on` and `dstaged` say whether they are used.
+// p and d always point into the LDS array; `on` and `dstaged` say whether they
+// are used.
 struct KRows {
-    double *p;          // K rows
-    const double *d;    // density rows
+    lds_double *p;          // K rows
+    const lds_double *d;    // density rows
     int width;          // doubles per row
     int loff;           // column of the first l AO
     int k_ao0, l_ao0;   // AOs of columns 0 and loff
@@ -778,8 +840,8 @@ __device__ __forceinline__ KRows make_krows(double *buf, int use_lds, int nrows,
     kr.width = kr.loff + w.l_nao;
     kr.k_ao0 = w.k_ao0;
     kr.l_ao0 = w.l_ao0;
-    kr.p = buf;
-    kr.d = buf + nrows * kr.width;
+    kr.p = (lds_double *)buf;
+    kr.d = kr.p + nrows * kr.width;
     return kr;
 }
 
@@ -788,7 +850,7 @@ __device__ __forceinline__ void krows_load_d(const KRows &kr, int nfi, int nfj, 
                                              const JKBuildArgs &a, int tid, int nthreads)
 {
     if (!kr.dstaged) return;
-    double *d = kr.p + (nfi + nfj) * kr.width;
+    lds_double *d = kr.p + (nfi + nfj) * kr.width;
     const int n_all = (nfi + nfj) * kr.width;
     for (int n = tid; n < n_all; n += nthreads) {
         int r = n / kr.width, c = n - r * kr.width;
@@ -1268,8 +1330,10 @@ CLASS_OCC2(3, 2, 3, 0)
 
 template <int LI, int LJ, int LK, int LL, int PM>
 __global__ __launch_bounds__(LANE_WAVES * WAVE, (ClassOcc<LI, LJ, LK, LL>::W))
-void jk_lane_kernel(JKBuildArgs a, int kl_chunk, int use_lds)
+void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
 {
+    int kl_chunk, use_lds;
+    const int item = select_task(a, batch, kl_chunk, use_lds);
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ);
     __shared__ uint32_t queue_all[LANE_WAVES][2][2 * WAVE];
     const int lane = threadIdx.x & (WAVE - 1);
@@ -1278,7 +1342,7 @@ void jk_lane_kernel(JKBuildArgs a, int kl_chunk, int use_lds)
     uint32_t *queue32 = queue_all[wid][1];
     const int nbas = a.nbas, nao = a.nao;
     select_replica(a);
-    WorkItem wi = work_item(a, kl_chunk, use_lds);
+    WorkItem wi = work_item(a, item, kl_chunk, use_lds);
     const uint32_t bas_ij = a.pairs_ij[wi.pij];
     const float q_ij = a.q_ij[wi.pij];
     const float kl_cutoff = a.cutoff - q_ij;
@@ -1408,8 +1472,10 @@ template <int LI, int LJ, int LK, int LL>
 __global__ __launch_bounds__((TeamShape<LI, LJ, LK, LL>::TB),
                              (TEAM_MIN_WAVES > ClassOcc<LI, LJ, LK, LL>::W ?
                               TEAM_MIN_WAVES : ClassOcc<LI, LJ, LK, LL>::W))
-void jk_team_kernel(JKBuildArgs a, int kl_chunk, int use_lds)
+void jk_team_kernel(JKBuildArgs a, TaskBatch batch)
 {
+    int kl_chunk, use_lds;
+    const int item = select_task(a, batch, kl_chunk, use_lds);
     using S = TeamShape<LI, LJ, LK, LL>;
     constexpr int NFI = S::NFI, NFJ = S::NFJ, NFK = S::NFK, NFL = S::NFL;
     constexpr int NROWS = S::NROWS, NFKL = S::NFKL, N = S::N, GS = S::GS;
@@ -1436,7 +1502,7 @@ void jk_team_kernel(JKBuildArgs a, int kl_chunk, int use_lds)
     const int nbas = a.nbas, nao = a.nao;
     const size_t nao2 = (size_t)nao * nao;
     select_replica(a);
-    WorkItem wi = work_item(a, kl_chunk, use_lds);
+    WorkItem wi = work_item(a, item, kl_chunk, use_lds);
     const uint32_t bas_ij = a.pairs_ij[wi.pij];
     const float kl_cutoff = a.cutoff - a.q_ij[wi.pij];
     if (a.q_kl[wi.kl0] + a.dm_penalty + Q_COND_MARGIN < kl_cutoff) return;
@@ -1764,114 +1830,12 @@ void jk_team_kernel(JKBuildArgs a, int kl_chunk, int use_lds)
     if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
 }
 
-// ---------------------------------------------------------------- dispatch
-// LDS bytes a workgroup may use (static + dynamic): the device limit, capped
-// at 64 KB.  gfx950 reports 160 KB per workgroup, but every launch of this
-// library stays within the 64 KB that has been validated on the hardware.
-#define JK_LDS_CAP (64 * 1024)
-static size_t lds_limit()
-{
-    static int cached_dev = -1;
-    static size_t cached = 0;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return JK_LDS_CAP;
-    if (dev != cached_dev) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess
-            || v <= 0 || v > JK_LDS_CAP)
-            v = JK_LDS_CAP;
-        cached = (size_t)v;
-        cached_dev = dev;
-    }
-    return cached;
-}
-
-// LDS K rows for a launch: 2 = K_ik/K_jk and K_il/K_jl, 1 = K_il/K_jl only,
-// 0 = none (several densities, no K, or too little LDS); `bytes` receives
-// the dynamic LDS size.  max_mode 1 suits kernels whose many short work
-// items would spend more on zeroing and flushing the wider rows (and on the
-// occupancy they cost) than the K_ik/K_jk atomics they save.
-// k_nao / l_nao: the K-row columns of a work item (the whole k and l groups
-// of the task, or with kl column windows the widest window, l_nao = 0 and
-// k_nao = kl_win_width).
-template <int LI, int LJ>
-static int krows_mode(const JKBuildArgs &a, int k_nao, int l_nao, size_t lds_static,
-                      int max_mode, bool drows, size_t &bytes)
-{
-    constexpr size_t NFIJ = ncart(LI) + ncart(LJ);
-    bytes = 0;
-    if (!a.vk || a.n_dm != 1 || l_nao < 0 || k_nao < 0 || k_nao + l_nao <= 0) return 0;
-    const size_t both = NFIJ * (size_t)(k_nao + l_nao) * sizeof(double);
-    const size_t lonly = NFIJ * (size_t)l_nao * sizeof(double);
-    if (max_mode >= 2 && drows && 2 * both + lds_static <= lds_limit()) {
-        bytes = 2 * both;
-        return 2 | KR_DROWS;
-    }
-    if (max_mode >= 2 && both + lds_static <= lds_limit()) { bytes = both; return 2; }
-    if (max_mode >= 1 && l_nao > 0 && lonly + lds_static <= lds_limit()) {
-        bytes = lonly;
-        return 1;
-    }
-    return 0;
-}
-
-// LDS K rows of a per-lane launch.  Candidates: the rows over the whole k and
-// l groups and, when the task has kl column windows, over one window, each
-// with and without the density rows.  Ranked by the rows kept in LDS (all
-// four K blocks, then K_il/K_jl only, then none), then by the workgroups a
-// CU can hold with that LDS (hipOccupancyMaxActiveBlocksPerMultiprocessor,
-// which also counts the kernel's registers), then whole groups before
-// windows, then with density rows before without.  kl_win_policy 1 takes the
-// windows whenever their rows fit.
-struct KrChoice { int use_lds; size_t bytes; };
-
-static KrChoice lane_krows_choice(const JKBuildArgs &a, size_t lds_static, bool win_ok,
-                                  const void *kernel, int nfij)
-{
-    KrChoice best{0, 0};
-    long best_key = -1;
-    const bool have_win = a.kl_win[0].win && win_ok && LANE_KROWS >= 2;
-    for (int win = 0; win < (have_win ? 2 : 1); ++win) {
-        const int kn = win ? a.kl_win[0].width : a.k_nao, ln = win ? 0 : a.l_nao;
-        for (int dr = (LANE_DROWS ? 1 : 0); dr >= 0; --dr) {
-            size_t bytes = 0;
-            // the generic krows_mode with this candidate's columns
-            int mode = 0;
-            if (a.vk && a.n_dm == 1 && kn + ln > 0) {
-                const size_t both = (size_t)nfij * (kn + ln) * sizeof(double);
-                const size_t lonly = (size_t)nfij * ln * sizeof(double);
-                if (LANE_KROWS >= 2 && dr && 2 * both + lds_static <= lds_limit()) {
-                    mode = 2 | KR_DROWS; bytes = 2 * both;
-                } else if (LANE_KROWS >= 2 && !dr && both + lds_static <= lds_limit()) {
-                    mode = 2; bytes = both;
-                } else if (!win && LANE_KROWS >= 1 && ln > 0 && lonly + lds_static <= lds_limit()) {
-                    mode = 1; bytes = lonly;
-                }
-            }
-            if (win && (mode & KR_MODE_MASK) != 2) continue;
-            int nb = 1;
-#if LANE_KROWS_OCC
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, LANE_WAVES * WAVE,
-                                                             bytes) != hipSuccess || nb < 1)
-                nb = 1;
-#endif
-            long key = ((long)(mode & KR_MODE_MASK) << 24) | ((long)nb << 8) |
-                       ((win ? 0 : 1) << 1) | (dr ? 1 : 0);
-            if (a.kl_win_policy == 1 && win) key |= 1L << 30;
-            if (key > best_key) {
-                best_key = key;
-                best.use_lds = mode | (win ? KR_WIN : 0);
-                best.bytes = bytes;
-            }
-        }
-    }
-    return best;
-}
-
+// ---------------------------------------------------------------- class info
 template <int LI, int LJ, int LK, int LL>
 struct ClassTraits {
     static constexpr int NF = ncart(LI) * ncart(LJ) * ncart(LK) * ncart(LL);
     static constexpr int GS = (LI+1)*(LJ+1)*(LK+1)*(LL+1);
+    static constexpr int N = (LI + LJ + LK + LL) / 2 + 1;
     // per-lane path when the block and three 2D tables fit in LANE_MAX doubles,
     // or when chunks of at most LANE_MAX_CHUNKS row blocks of the block do
     static constexpr bool LANE = (NF + 3 * GS <= LANE_MAX ||
@@ -1881,83 +1845,47 @@ struct ClassTraits {
                                  NF != LANE_SKIP_NF;
 };
 
-// one per-lane launch of precision mode PM (whole kl chunks or windows, as
-// lane_krows_choice ranks them for that kernel)
-template <int LI, int LJ, int LK, int LL, int PM>
-static hipError_t launch_lane(const JKBuildArgs &a, hipStream_t stream, long nblocks,
-                              int kl_chunk)
-{
-    const size_t lds_static = sizeof(uint32_t) * LANE_WAVES * 2 * 2 * WAVE;
-    const long nblocks_w = a.kl_win[0].win ? (long)a.npairs_ij * a.kl_win[0].n_win : 0;
-    const KrChoice c = lane_krows_choice(a, lds_static, nblocks_w <= 0x7fffffffL,
-                                         (const void *)jk_lane_kernel<LI, LJ, LK, LL, PM>,
-                                         ncart(LI) + ncart(LJ));
-    if (c.use_lds & KR_WIN) {
-        // K rows over one kl column window per work item
-        JKBuildArgs aw = a;
-        aw.pairs_kl = a.kl_win[0].pairs;
-        aw.q_kl = a.kl_win[0].q;
-        aw.pdata_kl = a.kl_win[0].pdata;
-        hipLaunchKernelGGL((jk_lane_kernel<LI, LJ, LK, LL, PM>), dim3(nblocks_w),
-                           dim3(LANE_WAVES * WAVE), c.bytes, stream, aw, 0, c.use_lds);
-    } else {
-        hipLaunchKernelGGL((jk_lane_kernel<LI, LJ, LK, LL, PM>), dim3(nblocks),
-                           dim3(LANE_WAVES * WAVE), c.bytes, stream, a, kl_chunk, c.use_lds);
-    }
-    return hipGetLastError();
-}
+// What the launcher (jk_launch.hip) needs to know of one class's kernel.
+#define JK_MAX_DEVICES 64
+struct ClassInfo {
+    bool lane;
+    const void *fn[2];          // mixed precision / FP64 only (the same for teams)
+    int threads;
+    size_t lds_static;
+    int nfij;                   // rows of the K rows
+    double cost;                // rough work of one primitive quartet
+    // workgroups per CU without dynamic LDS, per device (0: not yet asked);
+    // a property of the compiled kernel
+    std::atomic<int> *occ[2];
+};
 
 template <int LI, int LJ, int LK, int LL>
-static hipError_t launch_class(const JKBuildArgs &a, hipStream_t stream)
+static const ClassInfo *class_info()
 {
-    if constexpr (ClassTraits<LI, LJ, LK, LL>::LANE) {
-        // whole kl lists per work item unless that leaves the GPU idle
-        int nchunks = (LANE_ITEMS + a.npairs_ij - 1) / a.npairs_ij;
-        int maxchunks = (a.npairs_kl + LANE_MIN_CHUNK - 1) / LANE_MIN_CHUNK;
-        if (nchunks > maxchunks) nchunks = maxchunks;
-        if (nchunks < 1) nchunks = 1;
-        const int kl_chunk = (a.npairs_kl + nchunks - 1) / nchunks;
-        nchunks = (a.npairs_kl + kl_chunk - 1) / kl_chunk;
-        long nblocks = (long)a.npairs_ij * nchunks;
-        if (nblocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
-        // mixed precision: one kernel with both queues; FP64 only: the kernel
-        // compiled without the FP32 arithmetic
-        if (a.fp32_cut > -1e29f)
-            return launch_lane<LI, LJ, LK, LL, 0>(a, stream, nblocks, kl_chunk);
-        return launch_lane<LI, LJ, LK, LL, 1>(a, stream, nblocks, kl_chunk);
-    } else {
-        using S = TeamShape<LI, LJ, LK, LL>;
-        const int kl_chunk = TEAM_KL_CHUNK;
-        int nchunks = (a.npairs_kl + kl_chunk - 1) / kl_chunk;
-        long nblocks = (long)a.npairs_ij * nchunks;
-        if (nblocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
-        // static LDS of the kernel: queue, wave counts, stop flag, team buffers
-        size_t lds_static = sizeof(uint32_t) * 2 * S::TB + sizeof(int) * (S::TB / WAVE + 2) +
-                            sizeof(double) * (S::NQ * (S::PER_QB + S::DSZ) + S::NFI * S::NFJ) +
-                            256;
-        const JKWindows &tw = a.kl_win[1];
-        if (tw.win && a.vk && a.n_dm == 1 && (TEAM_KWIN || a.kl_win_policy == 1)) {
-            // K rows over one kl column window per work item, when that
-            // leaves enough work items to fill the GPU
-            const size_t bytes = sizeof(double) * (S::NFI + S::NFJ) * (size_t)tw.width;
-            const long nblocks_w = (long)a.npairs_ij * tw.n_win;
-            if (bytes + lds_static <= lds_limit() && nblocks_w <= 0x7fffffffL &&
-                (a.kl_win_policy == 1 || nblocks_w >= TEAM_KWIN_MIN_ITEMS)) {
-                JKBuildArgs aw = a;
-                aw.kl_win[0] = tw;
-                aw.pairs_kl = tw.pairs;
-                aw.q_kl = tw.q;
-                aw.pdata_kl = tw.pdata;
-                hipLaunchKernelGGL((jk_team_kernel<LI, LJ, LK, LL>), dim3(nblocks_w), dim3(S::TB),
-                                   bytes, stream, aw, 0, 2 | KR_WIN);
-                return hipGetLastError();
-            }
+    static std::atomic<int> occ[2][JK_MAX_DEVICES];
+    using T = ClassTraits<LI, LJ, LK, LL>;
+    static const ClassInfo info = [] {
+        ClassInfo c;
+        c.lane = T::LANE;
+        c.nfij = ncart(LI) + ncart(LJ);
+        c.cost = T::N * (3. * T::NF + 9. * T::GS) + 200.;
+        c.occ[0] = occ[0];
+        c.occ[1] = occ[1];
+        if constexpr (T::LANE) {
+            c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0>;
+            c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1>;
+            c.threads = LANE_WAVES * WAVE;
+            c.lds_static = sizeof(uint32_t) * LANE_WAVES * 2 * 2 * WAVE;
+        } else {
+            using S = TeamShape<LI, LJ, LK, LL>;
+            c.fn[0] = c.fn[1] = (const void *)jk_team_kernel<LI, LJ, LK, LL>;
+            c.threads = S::TB;
+            // queue, wave counts, stop flag, team buffers
+            c.lds_static = sizeof(uint32_t) * 2 * S::TB + sizeof(int) * (S::TB / WAVE + 2) +
+                           sizeof(double) * (S::NQ * (S::PER_QB + S::DSZ) + S::NFI * S::NFJ) +
+                           256;
         }
-        size_t lds = 0;
-        const int use_lds = krows_mode<LI, LJ>(a, a.k_nao, a.l_nao, lds_static, TEAM_KROWS,
-                                               false, lds);
-        hipLaunchKernelGGL((jk_team_kernel<LI, LJ, LK, LL>), dim3(nblocks), dim3(S::TB),
-                           lds, stream, a, kl_chunk, use_lds);
-    }
-    return hipGetLastError();
+        return c;
+    }();
+    return &info;
 }

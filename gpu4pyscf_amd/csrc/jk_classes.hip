@@ -13,21 +13,22 @@ static constexpr bool in_part(int li, int lj)
 }
 
 template <int I, int J, int K, int L>
-static hipError_t launch_if_in_part(const JKBuildArgs &a, hipStream_t stream)
+static const ClassInfo *info_if_in_part()
 {
-    if constexpr (in_part(I, J)) return launch_class<I, J, K, L>(a, stream);
-    else return hipErrorNotSupported;
+    if constexpr (in_part(I, J)) return class_info<I, J, K, L>();
+    else return nullptr;
 }
 
 #define JK_CASE(I, J, K, L) \
-    case ((I)*125 + (J)*25 + (K)*5 + (L)): return launch_if_in_part<I, J, K, L>(a, stream);
+    case ((I)*125 + (J)*25 + (K)*5 + (L)): return info_if_in_part<I, J, K, L>();
 
+#define JK_CASE_TYPE const ClassInfo *
 #include "jk_dispatch.inc"
 
 #define JK_CAT2(a, b) a##b
 #define JK_CAT(a, b) JK_CAT2(a, b)
 
-hipError_t JK_CAT(jk_dispatch_part, JK_PART)(int key, const JKBuildArgs &a, hipStream_t stream)
+const ClassInfo *JK_CAT(jk_class_info_part, JK_PART)(int key)
 {
-    return dispatch_class(key, a, stream);
+    return dispatch_class(key);
 }

@@ -3,7 +3,8 @@
 // instantiated by jk_classes.hip.
 #include <stdarg.h>
 #include <mutex>
-#include "jk_class_kernels.h"
+#include <new>
+#include "jk_launch.h"
 
 static thread_local char g_err[512];
 
@@ -18,35 +19,6 @@ static void set_err(const char *fmt, ...)
 void jk_set_error(const char *msg)
 {
     snprintf(g_err, sizeof(g_err), "%s", msg);
-}
-
-// class dispatch, one function per part of the class list (jk_classes.hip)
-hipError_t jk_dispatch_part0(int key, const JKBuildArgs &a, hipStream_t stream);
-hipError_t jk_dispatch_part1(int key, const JKBuildArgs &a, hipStream_t stream);
-hipError_t jk_dispatch_part2(int key, const JKBuildArgs &a, hipStream_t stream);
-hipError_t jk_dispatch_part3(int key, const JKBuildArgs &a, hipStream_t stream);
-hipError_t jk_dispatch_part4(int key, const JKBuildArgs &a, hipStream_t stream);
-
-// classes with a shell of l >= 4: the runtime-l kernels of jk_generic.hip
-hipError_t jk_dispatch_generic(const JKBuildArgs &a, hipStream_t stream);
-hipError_t jk_dispatch_generic_ip1(const JKBuildArgs &a, double *ejk, double jf, double kf,
-                                   hipStream_t stream);
-#define JK_TEMPLATED_LMAX 3
-
-static hipError_t dispatch(const JKBuildArgs &a, hipStream_t stream)
-{
-    if (a.li > JK_TEMPLATED_LMAX || a.lj > JK_TEMPLATED_LMAX || a.lk > JK_TEMPLATED_LMAX ||
-        a.ll > JK_TEMPLATED_LMAX)
-        return jk_dispatch_generic(a, stream);
-    const int key = a.li * 125 + a.lj * 25 + a.lk * 5 + a.ll;
-    hipError_t (*const parts[])(int, const JKBuildArgs &, hipStream_t) = {
-        jk_dispatch_part0, jk_dispatch_part1, jk_dispatch_part2, jk_dispatch_part3,
-        jk_dispatch_part4};
-    for (auto f : parts) {
-        hipError_t e = f(key, a, stream);
-        if (e != hipErrorNotSupported) return e;
-    }
-    return hipErrorNotSupported;
 }
 
 // ---------------------------------------------------------------- setup kernels
@@ -301,39 +273,6 @@ const char *jk_last_error(void) { return g_err; }
 
 int jk_abi_version(void) { return JK_ABI_VERSION; }
 
-int jk_build(const JKBuildArgs *args, void *stream);
-
-int jk_build_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks,
-                   void *const *streams, int nstreams)
-{
-    g_err[0] = 0;
-    if (!args || (ntasks > 0 && !tasks) || ntasks < 0 || nstreams < 1 || !streams) {
-        set_err("jk_build_tasks: null pointer or bad count (%d tasks)", ntasks);
-        return 1;
-    }
-    JKBuildArgs a = *args;
-    for (int m = 0; m < ntasks; ++m) {
-        const int t = ntasks - 1 - m;
-        const JKTask &k = tasks[t];
-        a.li = k.li; a.lj = k.lj; a.lk = k.lk; a.ll = k.ll;
-        a.iprim = k.iprim; a.jprim = k.jprim; a.kprim = k.kprim; a.lprim = k.lprim;
-        a.k_ao0 = k.k_ao0; a.k_nao = k.k_nao; a.l_ao0 = k.l_ao0; a.l_nao = k.l_nao;
-        a.npairs_ij = k.npairs_ij; a.npairs_kl = k.npairs_kl;
-        a.pairs_ij = k.pairs_ij; a.pairs_kl = k.pairs_kl;
-        a.q_ij = k.q_ij; a.q_kl = k.q_kl;
-        a.pdata_ij = k.pdata_ij; a.pdata_kl = k.pdata_kl;
-        a.kl_win[0] = k.kl_win[0];
-        a.kl_win[1] = k.kl_win[1];
-        a.swap_ijkl = k.swap_ijkl;
-        a.n_quartets = args->n_quartets ? args->n_quartets + t : nullptr;
-        a.n_quartets_fp32 = args->n_quartets_fp32 ? args->n_quartets_fp32 + t : nullptr;
-        a.quartet_hash = args->quartet_hash ? args->quartet_hash + t : nullptr;
-        const int st = jk_build(&a, streams[m % nstreams]);
-        if (st != 0) return st;
-    }
-    return 0;
-}
-
 // Host-side validation shared by jk_build and jk_energy_ip1; fills a copy
 // of the arguments with scale 0 taken as 1.  Returns 0 or a status code
 // (message set); -1: nothing to do (an empty pair list).
@@ -371,15 +310,42 @@ static int check_args(const JKBuildArgs *args, JKBuildArgs &a, const char *who)
     return 0;
 }
 
-int jk_build(const JKBuildArgs *args, void *stream)
+// the per-task fields of `k` into `a`
+static void set_task(JKBuildArgs &a, const JKTask &k)
 {
-    g_err[0] = 0;
-    JKBuildArgs a;
-    {
-        const int st = check_args(args, a, "jk_build");
-        if (st == -1) return 0;
-        if (st) return st;
-    }
+    a.li = k.li; a.lj = k.lj; a.lk = k.lk; a.ll = k.ll;
+    a.iprim = k.iprim; a.jprim = k.jprim; a.kprim = k.kprim; a.lprim = k.lprim;
+    a.k_ao0 = k.k_ao0; a.k_nao = k.k_nao; a.l_ao0 = k.l_ao0; a.l_nao = k.l_nao;
+    a.npairs_ij = k.npairs_ij; a.npairs_kl = k.npairs_kl;
+    a.pairs_ij = k.pairs_ij; a.pairs_kl = k.pairs_kl;
+    a.q_ij = k.q_ij; a.q_kl = k.q_kl;
+    a.pdata_ij = k.pdata_ij; a.pdata_kl = k.pdata_kl;
+    a.kl_win[0] = k.kl_win[0];
+    a.kl_win[1] = k.kl_win[1];
+    a.swap_ijkl = k.swap_ijkl;
+}
+
+static JKTask get_task(const JKBuildArgs &a)
+{
+    JKTask k;
+    k.li = a.li; k.lj = a.lj; k.lk = a.lk; k.ll = a.ll;
+    k.iprim = a.iprim; k.jprim = a.jprim; k.kprim = a.kprim; k.lprim = a.lprim;
+    k.k_ao0 = a.k_ao0; k.k_nao = a.k_nao; k.l_ao0 = a.l_ao0; k.l_nao = a.l_nao;
+    k.npairs_ij = a.npairs_ij; k.npairs_kl = a.npairs_kl;
+    k.pairs_ij = a.pairs_ij; k.pairs_kl = a.pairs_kl;
+    k.q_ij = a.q_ij; k.q_kl = a.q_kl;
+    k.pdata_ij = a.pdata_ij; k.pdata_kl = a.pdata_kl;
+    k.kl_win[0] = a.kl_win[0];
+    k.kl_win[1] = a.kl_win[1];
+    k.swap_ijkl = a.swap_ijkl;
+    return k;
+}
+
+// Validation of a J/K build task; as check_args.
+static int check_build(const JKBuildArgs *args, JKBuildArgs &a)
+{
+    const int st = check_args(args, a, "jk_build");
+    if (st) return st;
     if (!a.vj && !a.vk) { set_err("jk_build: neither vj nor vk given"); return 3; }
     if (a.screen < JK_SCREEN_JK || a.screen > JK_SCREEN_K ||
         (a.screen == JK_SCREEN_J && a.vk) || (a.screen == JK_SCREEN_K && a.vj)) {
@@ -396,25 +362,14 @@ int jk_build(const JKBuildArgs *args, void *stream)
         set_err("jk_build: Rys table lacks %d roots", nroots);
         return 3;
     }
-    hipError_t err = dispatch(a, (hipStream_t)stream);
-    if (err != hipSuccess) {
-        snprintf(g_err, sizeof(g_err), "jk_build (%d%d|%d%d): %s", a.li, a.lj, a.lk, a.ll,
-                 hipGetErrorString(err));
-        return 4;
-    }
     return 0;
 }
 
-int jk_energy_ip1(const JKBuildArgs *args, double *ejk, double j_factor, double k_factor,
-                  void *stream)
+// Validation of a gradient task; as check_args.
+static int check_ip1(const JKBuildArgs *args, JKBuildArgs &a, const double *ejk)
 {
-    g_err[0] = 0;
-    JKBuildArgs a;
-    {
-        const int st = check_args(args, a, "jk_energy_ip1");
-        if (st == -1) return 0;
-        if (st) return st;
-    }
+    const int st = check_args(args, a, "jk_energy_ip1");
+    if (st) return st;
     if (a.swap_ijkl) {
         set_err("jk_energy_ip1: swap_ijkl is for J/K builds only");
         return 3;
@@ -428,19 +383,103 @@ int jk_energy_ip1(const JKBuildArgs *args, double *ejk, double j_factor, double 
         set_err("jk_energy_ip1: Rys table lacks %d roots", nroots);
         return 3;
     }
-    // factors of the per-element two-particle density, as the reference's
-    // host code sets them (rys_contract_jk_ip1.cu:1789-1797): 8-fold
-    // symmetry times the 1/2 of the Coulomb energy for J, and the symmetric
-    // pair of exchange products for K, halved for a closed-shell density
-    if (a.n_dm == 1) k_factor *= .5;
-    const double jf = 4. * j_factor, kf = -2. * k_factor;
-    hipError_t err = jk_dispatch_generic_ip1(a, ejk, jf, kf, (hipStream_t)stream);
+    return 0;
+}
+
+// factors of the per-element two-particle density, as the reference's host
+// code sets them (rys_contract_jk_ip1.cu:1789-1797): 8-fold symmetry times the
+// 1/2 of the Coulomb energy for J, and the symmetric pair of exchange products
+// for K, halved for a closed-shell density
+static JKRun ip1_run(double *ejk, double j_factor, double k_factor, int n_dm)
+{
+    if (n_dm == 1) k_factor *= .5;
+    return JKRun{GEN_IP1, {ejk, 4. * j_factor, -2. * k_factor}};
+}
+
+static int launch(const char *who, const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                  void *const *streams, int nstreams, const JKRun &run)
+{
+    hipError_t err;
+    try {
+        err = jk_launch_tasks(a, tasks, ntasks, streams, nstreams, run);
+    } catch (const std::bad_alloc &) {
+        set_err("%s: out of host memory", who);
+        return 4;
+    }
     if (err != hipSuccess) {
-        snprintf(g_err, sizeof(g_err), "jk_energy_ip1 (%d%d|%d%d): %s", a.li, a.lj, a.lk, a.ll,
-                 hipGetErrorString(err));
+        set_err("%s: %s", who, hipGetErrorString(err));
         return 4;
     }
     return 0;
+}
+
+int jk_build(const JKBuildArgs *args, void *stream)
+{
+    g_err[0] = 0;
+    JKBuildArgs a;
+    const int st = check_build(args, a);
+    if (st == -1) return 0;
+    if (st) return st;
+    const JKTask k = get_task(a);
+    char who[64];
+    snprintf(who, sizeof(who), "jk_build (%d%d|%d%d)", a.li, a.lj, a.lk, a.ll);
+    return launch(who, a, &k, 1, &stream, 1, JKRun{GEN_JK, {nullptr, 0., 0.}});
+}
+
+int jk_build_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks,
+                   void *const *streams, int nstreams)
+{
+    g_err[0] = 0;
+    if (!args || (ntasks > 0 && !tasks) || ntasks < 0 || nstreams < 1 || !streams) {
+        set_err("jk_build_tasks: null pointer or bad count (%d tasks)", ntasks);
+        return 1;
+    }
+    JKBuildArgs in = *args, a = *args;
+    for (int t = ntasks - 1; t >= 0; --t) {
+        set_task(in, tasks[t]);
+        const int st = check_build(&in, a);
+        if (st > 0) return st;
+    }
+    return launch("jk_build_tasks", a, tasks, ntasks, streams, nstreams,
+                  JKRun{GEN_JK, {nullptr, 0., 0.}});
+}
+
+int jk_energy_ip1(const JKBuildArgs *args, double *ejk, double j_factor, double k_factor,
+                  void *stream)
+{
+    g_err[0] = 0;
+    JKBuildArgs a;
+    const int st = check_ip1(args, a, ejk);
+    if (st == -1) return 0;
+    if (st) return st;
+    a.n_repl = 1;
+    const JKTask k = get_task(a);
+    char who[64];
+    snprintf(who, sizeof(who), "jk_energy_ip1 (%d%d|%d%d)", a.li, a.lj, a.lk, a.ll);
+    return launch(who, a, &k, 1, &stream, 1, ip1_run(ejk, j_factor, k_factor, a.n_dm));
+}
+
+int jk_energy_ip1_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks, double *ejk,
+                        int n_copies, int64_t copy_stride, double j_factor, double k_factor,
+                        void *const *streams, int nstreams)
+{
+    g_err[0] = 0;
+    if (!args || (ntasks > 0 && !tasks) || ntasks < 0 || nstreams < 1 || !streams ||
+        n_copies < 1 || (n_copies > 1 && copy_stride < 3)) {
+        set_err("jk_energy_ip1_tasks: null pointer or bad count (%d tasks)", ntasks);
+        return 1;
+    }
+    JKBuildArgs in = *args, a = *args;
+    for (int t = ntasks - 1; t >= 0; --t) {
+        set_task(in, tasks[t]);
+        const int st = check_ip1(&in, a, ejk);
+        if (st > 0) return st;
+    }
+    a.n_repl = n_copies;
+    a.repl_stride = copy_stride;
+    a.vj = a.vk = nullptr;
+    return launch("jk_energy_ip1_tasks", a, tasks, ntasks, streams, nstreams,
+                  ip1_run(ejk, j_factor, k_factor, a.n_dm));
 }
 
 int jk_pair_data(double *out, const uint32_t *pairs, int npairs, int iprim,

@@ -1,0 +1,299 @@
+// Launch planning: the tasks of a build grouped by angular class into batched
+// launches (TaskBatch), spread over the caller's streams.
+#include <algorithm>
+#include <climits>
+#include <map>
+#include <mutex>
+#include <vector>
+#include "jk_launch.h"
+
+// class information, one function per part of the class list (jk_classes.hip)
+const ClassInfo *jk_class_info_part0(int key);
+const ClassInfo *jk_class_info_part1(int key);
+const ClassInfo *jk_class_info_part2(int key);
+const ClassInfo *jk_class_info_part3(int key);
+const ClassInfo *jk_class_info_part4(int key);
+
+#define JK_TEMPLATED_LMAX 3
+// LDS bytes a workgroup may use (static + dynamic): the device limit, capped
+// at 64 KB.  gfx950 reports 160 KB per workgroup, but every launch of this
+// library stays within the 64 KB that has been validated on the hardware.
+#define JK_LDS_CAP (64 * 1024)
+// LDS of a gfx950 CU is handed out in units of this many bytes
+#define JK_LDS_UNIT 1280
+
+static const ClassInfo *class_info_of(int key)
+{
+    const ClassInfo *(*const parts[])(int) = {jk_class_info_part0, jk_class_info_part1,
+                                              jk_class_info_part2, jk_class_info_part3,
+                                              jk_class_info_part4};
+    for (auto f : parts)
+        if (const ClassInfo *c = f(key)) return c;
+    return nullptr;
+}
+
+struct DeviceLimits { int dev; size_t lds_block, lds_cu; int cus; };
+
+static DeviceLimits device_limits()
+{
+    static std::mutex mu;
+    static DeviceLimits known[JK_MAX_DEVICES];
+    DeviceLimits l = {-1, JK_LDS_CAP, 160 * 1024, 256};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= JK_MAX_DEVICES) return l;
+    std::lock_guard<std::mutex> lock(mu);
+    if (known[dev].cus == 0) {
+        int v = 0;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) ==
+                hipSuccess && v > 0 && v < JK_LDS_CAP)
+            l.lds_block = v;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) ==
+                hipSuccess && v > 0)
+            l.lds_cu = v;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+            v > 0)
+            l.cus = v;
+        l.dev = dev;
+        known[dev] = l;
+    }
+    return known[dev];
+}
+
+// Workgroups per CU of a class kernel with `bytes` of dynamic LDS: by its
+// registers (asked once per kernel and device) and by the LDS of a CU.
+static int blocks_per_cu(const ClassInfo &c, int pm, size_t bytes, const DeviceLimits &lim)
+{
+    int nb = lim.dev >= 0 ? c.occ[pm][lim.dev].load(std::memory_order_relaxed) : 0;
+    if (nb == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, c.fn[pm], c.threads, 0) !=
+                hipSuccess || nb < 1)
+            nb = 1;
+        if (lim.dev >= 0) c.occ[pm][lim.dev].store(nb, std::memory_order_relaxed);
+    }
+    const size_t lds = (c.lds_static + bytes + JK_LDS_UNIT - 1) / JK_LDS_UNIT * JK_LDS_UNIT;
+    const int by_lds = (int)(lim.lds_cu / lds);
+    return std::max(1, std::min(nb, by_lds));
+}
+
+// One task of a launch.
+struct Item {
+    TaskDesc d;
+    long blocks;
+    size_t lds;
+    int per_cu;         // workgroups per CU with this LDS
+    double cost;        // rough work of the task
+};
+
+// LDS K rows of a per-lane task.  Candidates: the rows over the whole k and
+// l groups and, when the task has kl column windows, over one window, each
+// with and without the density rows.  Ranked by the rows kept in LDS (all
+// four K blocks, then K_il/K_jl only, then none), then by the workgroups a
+// CU can hold with that LDS, then whole groups before windows, then with
+// density rows before without.  kl_win_policy 1 takes the windows whenever
+// their rows fit.
+static void plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int pm,
+                      const DeviceLimits &lim, Item &it)
+{
+    // whole kl lists per work item unless that leaves the GPU idle
+    int nchunks = (LANE_ITEMS + k.npairs_ij - 1) / k.npairs_ij;
+    const int maxchunks = (k.npairs_kl + LANE_MIN_CHUNK - 1) / LANE_MIN_CHUNK;
+    nchunks = std::max(1, std::min(nchunks, maxchunks));
+    it.d.kl_chunk = (k.npairs_kl + nchunks - 1) / nchunks;
+    nchunks = (k.npairs_kl + it.d.kl_chunk - 1) / it.d.kl_chunk;
+    it.blocks = (long)k.npairs_ij * nchunks;
+    it.d.use_lds = 0;
+    it.lds = 0;
+    const JKWindows &w = k.kl_win[0];
+    const long blocks_w = w.win ? (long)k.npairs_ij * w.n_win : 0;
+    const bool have_win = w.win && blocks_w <= INT_MAX && LANE_KROWS >= 2;
+    long best_key = -1;
+    for (int win = 0; win < (have_win ? 2 : 1); ++win) {
+        const int kn = win ? w.width : k.k_nao, ln = win ? 0 : k.l_nao;
+        for (int dr = (LANE_DROWS ? 1 : 0); dr >= 0; --dr) {
+            size_t bytes = 0;
+            int mode = 0;
+            if (a.vk && a.n_dm == 1 && kn >= 0 && ln >= 0 && kn + ln > 0) {
+                const size_t both = (size_t)c.nfij * (kn + ln) * sizeof(double);
+                const size_t lonly = (size_t)c.nfij * ln * sizeof(double);
+                if (LANE_KROWS >= 2 && dr && 2 * both + c.lds_static <= lim.lds_block) {
+                    mode = 2 | KR_DROWS; bytes = 2 * both;
+                } else if (LANE_KROWS >= 2 && !dr && both + c.lds_static <= lim.lds_block) {
+                    mode = 2; bytes = both;
+                } else if (!win && LANE_KROWS >= 1 && ln > 0 &&
+                           lonly + c.lds_static <= lim.lds_block) {
+                    mode = 1; bytes = lonly;
+                }
+            }
+            if (win && (mode & KR_MODE_MASK) != 2) continue;
+            const int nb = blocks_per_cu(c, pm, bytes, lim);
+            long key = ((long)(mode & KR_MODE_MASK) << 24) | ((long)nb << 8) |
+                       ((win ? 0 : 1) << 1) | (dr ? 1 : 0);
+            if (a.kl_win_policy == 1 && win) key |= 1L << 30;
+            if (key > best_key) {
+                best_key = key;
+                it.d.use_lds = mode | (win ? KR_WIN : 0);
+                it.lds = bytes;
+                it.per_cu = nb;
+            }
+        }
+    }
+    if (it.d.use_lds & KR_WIN) {
+        it.d.pairs_kl = w.pairs; it.d.q_kl = w.q; it.d.pdata_kl = w.pdata; it.d.win = w.win;
+        it.blocks = blocks_w;
+    }
+}
+
+static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
+                      const DeviceLimits &lim, Item &it)
+{
+    it.d.kl_chunk = TEAM_KL_CHUNK;
+    it.blocks = (long)k.npairs_ij * ((k.npairs_kl + TEAM_KL_CHUNK - 1) / TEAM_KL_CHUNK);
+    it.d.use_lds = 0;
+    it.lds = 0;
+    const JKWindows &w = k.kl_win[1];
+    if (w.win && a.vk && a.n_dm == 1 && (TEAM_KWIN || a.kl_win_policy == 1)) {
+        // K rows over one kl column window per work item, when that leaves
+        // enough work items to fill the GPU
+        const size_t bytes = sizeof(double) * c.nfij * (size_t)w.width;
+        const long blocks_w = (long)k.npairs_ij * w.n_win;
+        if (bytes + c.lds_static <= lim.lds_block && blocks_w <= INT_MAX &&
+            (a.kl_win_policy == 1 || blocks_w >= TEAM_KWIN_MIN_ITEMS)) {
+            it.d.pairs_kl = w.pairs; it.d.q_kl = w.q; it.d.pdata_kl = w.pdata; it.d.win = w.win;
+            it.d.use_lds = 2 | KR_WIN;
+            it.blocks = blocks_w;
+            it.lds = bytes;
+        }
+    }
+    if (!(it.d.use_lds & KR_WIN) && TEAM_KROWS >= 1 && a.vk && a.n_dm == 1 && k.l_nao > 0) {
+        const size_t bytes = sizeof(double) * c.nfij * (size_t)k.l_nao;
+        if (bytes + c.lds_static <= lim.lds_block) { it.d.use_lds = 1; it.lds = bytes; }
+    }
+    it.per_cu = blocks_per_cu(c, 1, it.lds, lim);
+}
+
+// A kernel of this library and how it is launched.
+struct Kernel {
+    const void *fn;
+    int threads;
+};
+
+struct Launch {
+    Kernel k;
+    TaskBatch b;
+    long blocks;
+    size_t lds;
+    double cost;
+};
+
+// Cuts the items of one kernel into launches.  Items with the same LDS need go
+// together; others only join when the whole class leaves CUs idle anyway,
+// so that no item is held to the workgroups per CU of a wider one.
+static void make_launches(std::vector<Item> &items, const Kernel &kernel, int cus,
+                          std::vector<Launch> &out)
+{
+    long total = 0;
+    int per_cu = INT_MAX;
+    for (const Item &it : items) {
+        total += it.blocks;
+        per_cu = std::min(per_cu, it.per_cu);
+    }
+    const bool merge = total <= (long)cus * per_cu;
+    // the longest work items first: they start first, the short ones fill
+    // the tail
+    std::stable_sort(items.begin(), items.end(), [&](const Item &x, const Item &y) {
+        if (!merge && x.per_cu != y.per_cu) return x.per_cu < y.per_cu;
+        return x.cost / x.blocks > y.cost / y.blocks;
+    });
+    int last_cu = 0;
+    for (const Item &it : items) {
+        if (last_cu == 0 || out.back().b.n == JK_BATCH || (!merge && it.per_cu != last_cu) ||
+            out.back().blocks + it.blocks > INT_MAX) {
+            out.push_back(Launch());
+            Launch &l = out.back();
+            l.k = kernel;
+            l.b.n = l.b.pad = 0;
+            std::fill(l.b.block0, l.b.block0 + JK_BATCH + 1, INT_MAX);
+            l.blocks = 0;
+            l.lds = 0;
+            l.cost = 0.;
+        }
+        last_cu = it.per_cu;
+        Launch &l = out.back();
+        l.b.t[l.b.n] = it.d;
+        l.b.block0[l.b.n++] = (int)l.blocks;
+        l.blocks += it.blocks;
+        l.lds = std::max(l.lds, it.lds);
+        l.cost += it.cost;
+    }
+}
+
+hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                           void *const *streams, int nstreams, const JKRun &run)
+{
+    const DeviceLimits lim = device_limits();
+    const int pm = a.fp32_cut > -1e29f ? 0 : 1;
+    // items by kernel, the classes of the last tasks (f shells) first; the
+    // key of the runtime-l kernel is -1
+    struct Group { Kernel k; std::vector<Item> items; };
+    std::map<int, Group> by_kernel;
+    std::vector<int> order;
+    for (int t = ntasks - 1; t >= 0; --t) {
+        const JKTask &k = tasks[t];
+        if (k.npairs_ij <= 0 || k.npairs_kl <= 0) continue;
+        Item it;
+        TaskDesc &d = it.d;
+        d.pairs_ij = k.pairs_ij; d.pairs_kl = k.pairs_kl;
+        d.q_ij = k.q_ij; d.q_kl = k.q_kl;
+        d.pdata_ij = k.pdata_ij; d.pdata_kl = k.pdata_kl;
+        d.win = nullptr;
+        d.npairs_ij = k.npairs_ij; d.npairs_kl = k.npairs_kl;
+        d.prims_ij = k.iprim | (uint32_t)k.jprim << 16;
+        d.prims_kl = k.kprim | (uint32_t)k.lprim << 16;
+        d.k_ao0 = k.k_ao0; d.k_nao = k.k_nao; d.l_ao0 = k.l_ao0; d.l_nao = k.l_nao;
+        d.counter = t;
+        d.ls_swap = k.li | k.lj << 4 | k.lk << 8 | k.ll << 12 | (k.swap_ijkl != 0) << 16;
+        d.use_lds = 0;
+        const double quartets = (double)k.npairs_ij * k.npairs_kl * k.iprim * k.jprim * k.kprim *
+                                k.lprim;
+        int key = k.li * 125 + k.lj * 25 + k.lk * 5 + k.ll;
+        const bool small = k.li <= JK_TEMPLATED_LMAX && k.lj <= JK_TEMPLATED_LMAX &&
+                           k.lk <= JK_TEMPLATED_LMAX && k.ll <= JK_TEMPLATED_LMAX;
+        Kernel kern;
+        if (run.mode != GEN_JK || !small) {
+            key = -1;
+            kern = {jk_generic_kernel_of(run.mode), GEN_TB};
+            if (!jk_generic_plan(k, run.mode, d, it.blocks, it.lds)) return hipErrorNotSupported;
+            it.per_cu = (int)(lim.lds_cu / (it.lds + 4096));
+            it.cost = quartets * ncart(k.li) * ncart(k.lj) * ncart(k.lk) * ncart(k.ll);
+        } else {
+            const ClassInfo *c = class_info_of(key);
+            if (!c) return hipErrorNotSupported;
+            kern = {c->fn[pm], c->threads};
+            if (c->lane) plan_lane(a, k, *c, pm, lim, it);
+            else plan_team(a, k, *c, lim, it);
+            it.cost = quartets * c->cost;
+        }
+        if (it.blocks > INT_MAX) return hipErrorInvalidConfiguration;
+        Group &g = by_kernel[key];
+        if (g.items.empty()) {
+            order.push_back(key);
+            g.k = kern;
+        }
+        g.items.push_back(it);
+    }
+    std::vector<Launch> launches;
+    for (int key : order)
+        make_launches(by_kernel[key].items, by_kernel[key].k, lim.cus, launches);
+    // each launch on the stream with the least work so far
+    std::vector<double> load(nstreams, 0.);
+    for (Launch &l : launches) {
+        const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        load[s] += l.cost;
+        void *args[] = {(void *)&a, &l.b, (void *)&run.ex};
+        const hipError_t err = hipLaunchKernel(l.k.fn, dim3((unsigned)l.blocks),
+                                               dim3(l.k.threads), args, l.lds,
+                                               (hipStream_t)streams[s]);
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
+}

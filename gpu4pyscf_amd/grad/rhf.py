@@ -22,6 +22,8 @@ __all__ = ['_jk_energy_per_atom', '_VHFOpt']
 
 _VHFOpt = jk_mod._VHFOpt
 
+EJK_COPIES = 64
+
 
 def _jk_energy_per_atom(vhfopt, dm, j_factor=1., k_factor=1., omega=None, lr_factor=None,
                         sr_factor=None, verbose=None):
@@ -51,7 +53,8 @@ def _jk_energy_per_atom(vhfopt, dm, j_factor=1., k_factor=1., omega=None, lr_fac
                               ctypes.c_int(n_dm), ctypes.c_int(nao), jk_mod._ptr(d['ao_loc']),
                               ctypes.c_int(nbas), ctypes.c_int(1), stream), 'jk_dm_cond')
     natm = vhfopt.mol.natm
-    ejk = torch.zeros((natm, 3), dtype=torch.float64, device=dms.device)
+    # copies of the natm x 3 result the workgroups add into
+    ejk = torch.zeros((EJK_COPIES, natm, 3), dtype=torch.float64, device=dms.device)
     args = clib.JKBuildArgs()
     args.abi_version = clib.JK_ABI_VERSION
     args.nbas, args.nao = nbas, nao
@@ -63,22 +66,13 @@ def _jk_energy_per_atom(vhfopt, dm, j_factor=1., k_factor=1., omega=None, lr_fac
     args.n_dm = n_dm
     args.dm = dms.data_ptr()
     args.rys = vhfopt._rys
-    args.n_repl = 1
-    args.repl_stride = dms.numel()
-    uniq = mol.uniq_l_ctr
-    passes = vhfopt.operator_passes(omega)
-    for (i, j, k, l) in vhfopt.tasks():
-        args.li, args.lj, args.lk, args.ll = (int(uniq[x, 0]) for x in (i, j, k, l))
-        args.iprim, args.jprim, args.kprim, args.lprim = (int(uniq[x, 1]) for x in (i, j, k, l))
-        pij, pkl = d['pairs'][i, j], d['pairs'][k, l]
-        args.npairs_ij, args.npairs_kl = len(pij), len(pkl)
-        args.pairs_ij, args.pairs_kl = pij.data_ptr(), pkl.data_ptr()
-        args.q_ij, args.q_kl = d['q'][i, j].data_ptr(), d['q'][k, l].data_ptr()
-        args.pdata_ij = d['pdata'][i, j].data_ptr()
-        args.pdata_kl = d['pdata'][k, l].data_ptr()
-        for w, f in passes:
+    tasks, ntasks = vhfopt.ip1_task_array()
+    with vhfopt.fork_streams(dms.device) as streams:
+        handles = (ctypes.c_void_p * len(streams))(*[s.cuda_stream for s in streams])
+        for w, f in vhfopt.operator_passes(omega):
             args.omega, args.scale = w, f
-            st = lib.jk_energy_ip1(ctypes.byref(args), ctypes.c_void_p(ejk.data_ptr()),
-                                   float(j_factor), float(k_factor), stream)
-            clib.check(st, f'jk_energy_ip1 {tuple(int(uniq[x, 0]) for x in (i, j, k, l))}')
-    return ejk.cpu().numpy()
+            clib.check(lib.jk_energy_ip1_tasks(
+                ctypes.byref(args), tasks, ntasks, ejk.data_ptr(), EJK_COPIES,
+                3 * natm, float(j_factor), float(k_factor), handles, len(streams)),
+                'jk_energy_ip1_tasks')
+    return ejk.sum(0).cpu().numpy()

@@ -117,7 +117,7 @@ class JKTask(ctypes.Structure):
 
 
 EXPORTS = ('jk_build', 'jk_build_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
-           'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_md_dm_to_hermite', 'jk_md_hermite_to_j',
+           'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_energy_ip1_tasks', 'jk_md_dm_to_hermite', 'jk_md_hermite_to_j',
            'jk_md_build_j', 'jk_int1e', 'jk_ao_transform', 'mlp_gemm_bf16', 'mlp_silu_backward', 'mlp_colsum', 'mlp_mse_grad',
            'mlp_adamw', 'mlp_to_bf16', 'jk_last_error', 'jk_abi_version')
 
@@ -135,7 +135,7 @@ def load():
     lib = ctypes.CDLL(LIB_PATH)
     lib.jk_last_error.restype = ctypes.c_char_p
     for name in ('jk_build', 'jk_build_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
-                 'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_abi_version'):
+                 'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_energy_ip1_tasks', 'jk_abi_version'):
         getattr(lib, name).restype = ctypes.c_int
     lib.jk_build.argtypes = [ctypes.POINTER(JKBuildArgs), c_void_p]
     lib.jk_md_build_j.restype = ctypes.c_int
@@ -148,6 +148,9 @@ def load():
                       c_void_p]
     lib.jk_energy_ip1.argtypes = [ctypes.POINTER(JKBuildArgs), c_void_p, ctypes.c_double,
                                   ctypes.c_double, c_void_p]
+    lib.jk_energy_ip1_tasks.argtypes = [ctypes.POINTER(JKBuildArgs), c_void_p, ctypes.c_int,
+                                        c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_double,
+                                        ctypes.c_double, c_void_p, ctypes.c_int]
     lib.jk_pair_qcond.argtypes = [c_void_p, c_void_p, ctypes.c_int, c_void_p, c_void_p,
                                   ctypes.c_int, JKRysTable, ctypes.c_double, ctypes.c_double,
                                   ctypes.c_double, c_void_p]

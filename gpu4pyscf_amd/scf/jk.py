@@ -16,6 +16,7 @@ sends l > 4 to PySCF on the CPU, gpu4pyscf/scf/jk.py:622-640; no CPU path
 exists here).
 '''
 
+import contextlib
 import ctypes
 import math
 import time
@@ -438,7 +439,46 @@ class _VHFOpt:
             self._fill_task(arr[t], d, task)
         return arr
 
-    def _fill_task(self, a, d, task):
+    def ip1_task_array(self):
+        '''(ctypes array of JKTask, count) of an energy gradient: the tasks of
+        the J/K build, none with bra and ket exchanged; built once per
+        geometry and task filter.'''
+        d = self._dev
+        tasks = self.tasks()
+        if d.get('ip1_tasks', (None,))[0] != tasks:
+            arr = (clib.JKTask * max(len(tasks), 1))()
+            for t, task in enumerate(tasks):
+                self._fill_task(arr[t], d, task, swap=False)
+            d['ip1_tasks'] = (tasks, arr)
+        return d['ip1_tasks'][1], len(tasks)
+
+    @contextlib.contextmanager
+    def fork_streams(self, device):
+        '''The caller's stream and nstreams - 1 side streams that wait for it;
+        joined back into it on exit, also when a launch failed, so that no
+        kernel still runs when its buffers are released.'''
+        torch = _torch()
+        cur = torch.cuda.current_stream(device)
+        streams = [cur]
+        if self.nstreams > 1:
+            key = str(device)
+            if key not in self._streams:
+                self._streams[key] = [torch.cuda.Stream(device)
+                                      for _ in range(self.nstreams - 1)]
+            streams += self._streams[key][:self.nstreams - 1]
+            ready = torch.cuda.Event()
+            ready.record(cur)
+            for s in streams[1:]:
+                s.wait_event(ready)
+        try:
+            yield streams
+        finally:
+            for s in streams[1:]:
+                done = torch.cuda.Event()
+                done.record(s)
+                cur.wait_event(done)
+
+    def _fill_task(self, a, d, task, swap=None):
         '''Per-task fields of a JKTask / JKBuildArgs for class task (i, j, k,
         l); with swap_tasks, the (xs|xp) tasks (li = lk, lj = 0, ll = 1; the
         two group pairs differ) run with bra and ket exchanged
@@ -452,8 +492,9 @@ class _VHFOpt:
         goff = mol.group_offsets
         ls = [int(uniq[x, 0]) for x in task]
         i, j, k, l = task
-        swap = (self.swap_tasks and (i, j) != (k, l) and ls[0] == ls[2] and
-                ls[1] == 0 and ls[3] == 1)
+        if swap is None:
+            swap = (self.swap_tasks and (i, j) != (k, l) and ls[0] == ls[2] and
+                    ls[1] == 0 and ls[3] == 1)
         if swap:
             i, j, k, l = k, l, i, j
         a.li, a.lj, a.lk, a.ll = (int(uniq[x, 0]) for x in (i, j, k, l))
@@ -593,33 +634,15 @@ class _VHFOpt:
         # launch passes of the operator: (omega, scale, with J, with K)
         runs = [(w, f, with_j, with_k)
                 for w, f in self.operator_passes(omega, lr_factor, sr_factor)]
-        cur = torch.cuda.current_stream(dms.device)
-        streams = [cur]
-        if self.nstreams > 1:
-            key = str(dms.device)
-            if key not in self._streams:
-                self._streams[key] = [torch.cuda.Stream(dms.device)
-                                      for _ in range(self.nstreams - 1)]
-            streams += self._streams[key][:self.nstreams - 1]
-            ready = torch.cuda.Event()
-            ready.record(cur)
-            for s in streams[1:]:
-                s.wait_event(ready)
-        # the side streams are joined back into the caller's stream even when a
-        # launch fails, so that no kernel still adds into vj/vk after they are
-        # released
-        try:
+        with self.fork_streams(dms.device) as streams:
             for n_run, (w, f, rj, rk) in enumerate(runs):
                 args.omega = w
                 args.scale = f
                 args.vj = vj.data_ptr() if rj else None
                 args.vk = vk.data_ptr() if rk else None
                 first = n_run == 0
-                # launched from the last task (f classes, the longest) to the
-                # first, so that the short s/p classes fill the streams at the
-                # end (32-water def2-TZVP build: 521 ms in task order, 515
-                # reversed).  Without per-launch timing the whole loop is one
-                # native call.
+                # one native call; with per-launch timing a launch per task,
+                # from the last (f classes, the longest) to the first
                 if not (time_classes or prof):
                     args.n_quartets = counter.data_ptr() if (first and counter is not None) else None
                     args.n_quartets_fp32 = (counter32.data_ptr()
@@ -649,11 +672,6 @@ class _VHFOpt:
                     if st != 0:
                         clib.check(st, f'jk_build ({"spdfghi"[args.li]}{"spdfghi"[args.lj]}|'
                                        f'{"spdfghi"[args.lk]}{"spdfghi"[args.ll]})')
-        finally:
-            for s in streams[1:]:
-                done = torch.cuda.Event()
-                done.record(s)
-                cur.wait_event(done)
         if with_j:
             vj = vj[0] if n_repl == 1 else vj.sum(0)
         if with_k:

@@ -191,14 +191,23 @@ typedef struct {
 
 /* All class tasks of one build: the task loop of gpu4pyscf/scf/jk.py:554-585
  * in one call.  *args supplies the fields shared by the tasks; tasks[t] the
- * per-task ones.  Tasks are launched from the last to the first, the m-th
- * launch on streams[m % nstreams] (hipStream_t; NULL entries are the null
- * stream).  When args->n_quartets, n_quartets_fp32 or quartet_hash is set it
- * points to ntasks counters and task t adds into element t.  Stops at and
- * returns the status of the first task that fails.  No counterpart in the
+ * per-task ones.  Tasks of one angular class go into common launches, the
+ * classes of the last tasks first, each launch on the stream (streams[0 ..
+ * nstreams), hipStream_t; NULL entries are the null stream) with the least
+ * estimated work so far.  When args->n_quartets, n_quartets_fp32 or quartet_hash is set it
+ * points to ntasks counters and task t adds into element t.  Every task is
+ * checked, from the last to the first, before the first launch.  No counterpart in the
  * reference, which calls RYS_build_jk once per task from Python. */
 int jk_build_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks,
                    void *const *streams, int nstreams);
+
+/* jk_energy_ip1 for all class tasks in one call, as jk_build_tasks; ejk:
+ * n_copies zeroed arrays of natm x 3, copy_stride doubles apart, whose sum is
+ * the result (the workgroups add into different copies, so that the few
+ * addresses are not fought over). */
+int jk_energy_ip1_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks, double *ejk,
+                        int n_copies, int64_t copy_stride, double j_factor, double k_factor,
+                        void *const *streams, int nstreams);
 
 /* ---- McMurchie-Davidson J-engine (basis of single-primitive shells,
  * SortedGTO(decontract=True)).  Replaces the reference's MD J path
