@@ -33,6 +33,10 @@ __device__ __forceinline__ bool survives_ejk(float q_kl, float kl_cutoff, uint32
 bool jk_generic_plan(const JKTask &k, int mode, TaskDesc &d, long &blocks, size_t &lds);
 const void *jk_generic_kernel_of(int mode);
 
+// the per-lane gradient kernel of a class (key: li*125 + lj*25 + lk*5 + ll),
+// one wavefront per workgroup, or NULL (jk_ip1.hip)
+const void *jk_ip1_lane_kernel_of(int key);
+
 // What a run of class tasks computes: J/K (GEN_JK) or the energy gradient.
 struct JKRun {
     int mode;

@@ -19,6 +19,8 @@ const ClassInfo *jk_class_info_part4(int key);
 // at 64 KB.  gfx950 reports 160 KB per workgroup, but every launch of this
 // library stays within the 64 KB that has been validated on the hardware.
 #define JK_LDS_CAP (64 * 1024)
+// work items per launch that the kl chunks of the per-lane gradient aim at
+#define IP1_ITEMS 4096
 // LDS of a gfx950 CU is handed out in units of this many bytes
 #define JK_LDS_UNIT 1280
 
@@ -258,8 +260,18 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
         int key = k.li * 125 + k.lj * 25 + k.lk * 5 + k.ll;
         const bool small = k.li <= JK_TEMPLATED_LMAX && k.lj <= JK_TEMPLATED_LMAX &&
                            k.lk <= JK_TEMPLATED_LMAX && k.ll <= JK_TEMPLATED_LMAX;
+        const void *ip1 = run.mode != GEN_JK && small ? jk_ip1_lane_kernel_of(key) : nullptr;
         Kernel kern;
-        if (run.mode != GEN_JK || !small) {
+        if (ip1) {
+            kern = {ip1, WAVE};
+            const int nchunks = std::min((IP1_ITEMS + k.npairs_ij - 1) / k.npairs_ij,
+                                         (k.npairs_kl + WAVE - 1) / WAVE);
+            d.kl_chunk = (k.npairs_kl + nchunks - 1) / nchunks;
+            it.blocks = (long)k.npairs_ij * ((k.npairs_kl + d.kl_chunk - 1) / d.kl_chunk);
+            it.lds = 0;
+            it.per_cu = 4;
+            it.cost = quartets * ncart(k.li) * ncart(k.lj) * ncart(k.lk) * ncart(k.ll);
+        } else if (run.mode != GEN_JK || !small) {
             key = -1;
             kern = {jk_generic_kernel_of(run.mode), GEN_TB};
             if (!jk_generic_plan(k, run.mode, d, it.blocks, it.lds)) return hipErrorNotSupported;
@@ -284,7 +296,9 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
     std::vector<Launch> launches;
     for (int key : order)
         make_launches(by_kernel[key].items, by_kernel[key].k, lim.cus, launches);
-    // each launch on the stream with the least work so far
+    // each launch on the stream with the least work so far, in class order
+    // (sorted by the estimate: 54 -> 60 ms on the 8-water two-density build;
+    // round-robin: the 16-water range-separated K 144 -> 148 ms)
     std::vector<double> load(nstreams, 0.);
     for (Launch &l : launches) {
         const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
