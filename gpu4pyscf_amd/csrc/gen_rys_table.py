@@ -27,10 +27,14 @@ unit intervals [k, k+1).  Output: rys_table.npz with
   coef[off[n-1] + (k*2n + f)*(DEGREE+1) + d]   f = 2i (root i), 2i+1 (weight i)
   xmax[n-1] = X_n, off[n-1], large_r[n*(n-1)/2 + i], large_w[...].
 
-For one to three roots the kernels instead take the moments F_0..F_{2n-1}
-from a Boys grid, boys[g, m] = F_m(g * BOYS_STEP) for m <= BOYS_M - 1, by
-the BOYS_TERMS-term Taylor series F_m(x) = sum_k F_{m+k}(x_g) (x_g - x)^k / k!
-about the nearest grid point, and form the Gauss rule from the moments.
+For one to three roots the kernels instead form the Gauss rule of the Boys
+moments F_0..F_{2n-1}.  Row g of moments{n} holds, for x_g = g * MOMENT_STEP and
+M = 2n - 1, F_{M+k}(x_g) / k! for k < MOMENT_TERMS, exp(-x_g) and one zero:
+F_M(x) = sum_k F_{M+k}(x_g) (x_g - x)^k / k! about the nearest row (the next term
+is below 1e-17 of it), exp(-x) = exp(-x_g) exp(x_g - x), and the lower moments by
+F_{m-1} = (2 x F_m + exp(-x)) / (2m - 1), whose terms are all positive.
+boys[g, m] = F_m(g * BOYS_STEP) is a finer grid of the moments themselves, kept
+for the tests.
 
 Run:  python gen_rys_table.py  (about a minute on 8 cores).
 '''
@@ -46,7 +50,19 @@ WIDTH = 1.0
 BOYS_STEP = 0.1
 BOYS_TERMS = 8
 BOYS_M = 5 + BOYS_TERMS        # F_0 .. F_12: moments of up to three roots
+MOMENT_STEP = 0.5
+MOMENT_TERMS = 12
 mp.mp.dps = 40
+
+
+def moment_rows(n, xmax):
+    '''Rows of moments{n}, covering x < xmax.'''
+    out = []
+    for g in range(int(xmax / MOMENT_STEP + .5) + 1):
+        f = boys(2*n - 2 + MOMENT_TERMS, g * MOMENT_STEP)
+        out.append([float(f[2*n - 1 + k] / mp.factorial(k)) for k in range(MOMENT_TERMS)] +
+                   [float(mp.exp(-mp.mpf(g) * MOMENT_STEP)), 0.])
+    return np.array(out)
 
 
 def boys(nmax, x):
@@ -194,7 +210,9 @@ def main(out):
     np.savez(out, coef=np.concatenate(coefs), off=np.asarray(offs, dtype=np.int64),
              xmax=np.asarray(xmax, dtype=np.float64), degree=DEGREE, width=WIDTH,
              nmax=NMAX, large_r=np.asarray(large_r), large_w=np.asarray(large_w),
-             boys=boys_grid, boys_step=BOYS_STEP, boys_terms=BOYS_TERMS)
+             boys=boys_grid, boys_step=BOYS_STEP, boys_terms=BOYS_TERMS,
+             moment_step=MOMENT_STEP,
+             **{f'moments{n}': moment_rows(n, xmax[n-1]) for n in (1, 2, 3)})
 
 
 if __name__ == '__main__':

@@ -29,7 +29,7 @@
 // read by the digestion staged in LDS; what remains per quartet (J_kl, and
 // K in the team kernel) goes to HBM with FP64 atomics.
 // Rys roots: for up to three roots the Gauss rule of Boys moments taken from
-// a Boys grid by a Taylor series; otherwise Chebyshev tables; both generated
+// Taylor series of one of them; otherwise Chebyshev tables; both generated
 // by gen_rys_table.py.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -44,11 +44,6 @@
 #define Q_COND_MARGIN   4.f
 #define WAVE            64
 #define RYS_DEG_MAX     15
-// the team kernel's one-root-per-lane evaluation uses the Boys-grid rule
-// (all roots, one kept) up to this many roots, the Chebyshev tables above
-#ifndef ROOT_ONE_BOYS_NMAX
-#define ROOT_ONE_BOYS_NMAX 2
-#endif
 // classes whose Cartesian block plus three 2D tables fit in LANE_MAX
 // doubles run one quartet per lane, the others on teams of lanes.
 // Measured (ms per 32-water def2-TZVP build): 120 -> 720, 150 -> 679,
@@ -333,65 +328,163 @@ __device__ __forceinline__ double seg_sum(double v, const SegMask &m)
     return v;
 }
 
-// Boys moments F_0..F_{NM-1}(x), x < xmax[2], by the 8-term Taylor series
-// about the nearest point x_g of the Boys grid:
-// F_m(x) = sum_k F_{m+k}(x_g) (x_g - x)^k / k!  (|x_g - x| <= step/2).
-template <int NM>
-__device__ __forceinline__ void boys_moments(const JKRysTable &tab, double x, double *f)
+// Reciprocal, quotient, reciprocal square root and square root of normal
+// numbers, within an ulp: the hardware estimates (24 bits) with two Newton
+// steps, 5 to 8 instructions where the IEEE forms take 10 to 20.
+__device__ __forceinline__ double rcp64(double x)
 {
-    constexpr double INV_FACT[8] = {1., 1., 1. / 2, 1. / 6, 1. / 24, 1. / 120, 1. / 720,
-                                    1. / 5040};
-    int g = (int)(x * tab.boys_inv_step + .5);
-    g = g < tab.boys_rows - 1 ? g : tab.boys_rows - 1;
-    const double d = g * tab.boys_step - x;
-    const double *F = tab.coef + tab.boys + (int64_t)g * JK_BOYS_M;
-    double Fg[NM + 7];
-#pragma unroll
-    for (int m = 0; m < NM + 7; ++m) Fg[m] = F[m];
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        double s = Fg[m + 7] * INV_FACT[7];
-#pragma unroll
-        for (int k = 6; k >= 0; --k) s = fma(s, d, Fg[m + k] * INV_FACT[k]);
-        f[m] = s;
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.), r, r);
+    return fma(fma(-x, r, 1.), r, r);
+}
+
+__device__ __forceinline__ double div64(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.), r, r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+
+__device__ __forceinline__ double rsqrt64(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(y, fma(-x * y, .5 * y, .5), y);
+    return fma(y, fma(-x * y, .5 * y, .5), y);
+}
+
+__device__ __forceinline__ double sqrt64(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(y, fma(-x * y, .5 * y, .5), y);
+    const double s = x * y;
+    return fma(fma(-s, s, x), .5 * y, s);
+}
+
+// the same for the FP32 quartets
+__device__ __forceinline__ float rcp64(float x) { return 1.f / x; }
+__device__ __forceinline__ float rsqrt64(float x) { return sqrtf(1.f / x); }
+
+// Moment rows of the N-point rule in LDS (JKRysTable.boys: N = 1, 2, 3), one
+// copy per workgroup.  A row is read whole by every lane at an address of its
+// own; from the caches such a gather occupies the address units for 64 lines,
+// and they were 65 to 80 % busy in the s and p classes ((ss|ss), (ps|ss),
+// (ps|ps)).  One Taylor series of the highest moment, one of the exponential
+// and a downward recursion replace a series per moment: 27 + 2N fused
+// operations against 32 N.  Rows of 14 doubles 0.5 apart keep the copy at 9 to
+// 12 KB (a grid of 0.1 for all moments took 56 KB, larger than the L1).
+// 48 waters (def2-TZVP): (fs|ps) 45.8 -> 37.2 ms, (fp|ps) 34.7 -> 31.7, (dp|ps)
+// 42.9 -> 40.6, the whole build 1019 -> 1000; 8 waters (def2-SVP) 2.91 -> 2.55.
+#define MOMENT_TERMS 12
+#define MOMENT_STEP .5
+__host__ __device__ constexpr int moment_rows(int n) { return n == 1 ? 79 : n == 2 ? 95 : n == 3 ? 109 : 0; }
+typedef double double2v __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) double2v lds_double2;
+
+template <int N>
+struct MomentRows {
+    static constexpr int SIZE = N <= 3 ? moment_rows(N) * JK_BOYS_M : 2;    // doubles
+};
+
+// copies the rows (a barrier must follow)
+template <int N>
+__device__ __forceinline__ void load_moment_rows(double *buf, const JKRysTable &tab, int tid,
+                                                 int nthreads)
+{
+    if constexpr (N <= 3) {
+        const int before = (N > 1 ? moment_rows(1) : 0) + (N > 2 ? moment_rows(2) : 0);
+        const double2v *src = (const double2v *)(tab.coef + tab.boys + before * JK_BOYS_M);
+        lds_double2 *dst = (lds_double2 *)(lds_double *)buf;
+        for (int n = tid; n < MomentRows<N>::SIZE / 2; n += nthreads) dst[n] = src[n];
     }
 }
 
-// Rys nodes u_i = t_i^2 and weights: the large-x limit above xmax[N-1];
-// below it, for one to three roots the Gauss rule of the Boys moments,
-// else the Chebyshev tables.
+// A constant that is put into scalar registers where it is used: left to
+// itself the compiler keeps the factorials of the two series in 24 vector
+// registers over the whole kernel ((ss|ss) 86 -> 124, (ps|ss) 119 -> 142).
+__device__ __forceinline__ double scalar_const(double c)
+{
+    asm volatile("" : "+s"(c));
+    return c;
+}
+
+// Boys moments F_0..F_{2N-1}(x), x < xmax[N-1]
 template <int N>
-__device__ __forceinline__ void rys_roots(const JKRysTable &tab, double x,
-                                          double *r, double *w)
+__device__ __forceinline__ void boys_moments(const lds_double *rows, double x, double *f)
+{
+    constexpr int M = 2 * N - 1;
+    constexpr double INV_FACT[13] = {1., 1., 1. / 2, 1. / 6, 1. / 24, 1. / 120, 1. / 720,
+                                     1. / 5040, 1. / 40320, 1. / 362880, 1. / 3628800,
+                                     1. / 39916800, 1. / 479001600};
+    int g = (int)fma(x, 1. / MOMENT_STEP, .5);
+    g = g < moment_rows(N) - 1 ? g : moment_rows(N) - 1;
+    const double d = fma((double)g, MOMENT_STEP, -x);
+    const lds_double2 *p = (const lds_double2 *)(rows + g * JK_BOYS_M);
+    double c[JK_BOYS_M];
+#pragma unroll
+    for (int k = 0; k < JK_BOYS_M / 2; ++k) {
+        const double2v v = p[k];
+        c[2 * k] = v.x; c[2 * k + 1] = v.y;
+    }
+    double s = c[MOMENT_TERMS - 1], e = scalar_const(INV_FACT[12]);
+#pragma unroll
+    for (int k = MOMENT_TERMS - 2; k >= 0; --k) s = fma(s, d, c[k]);
+#pragma unroll
+    for (int k = 11; k >= 0; --k)
+        e = fma(e, d, k > 2 ? scalar_const(INV_FACT[k]) : INV_FACT[k]);
+    e *= c[MOMENT_TERMS];
+    const double x2 = 2. * x;
+    f[M] = s;
+#pragma unroll
+    for (int m = M; m > 0; --m) f[m - 1] = fma(x2, f[m], e) * (1. / (2 * m - 1));
+}
+
+// Rys nodes u_i = t_i^2 and weights: the large-x limit above xmax[N-1]
+// (Gauss-Hermite); below it, for one to three roots the Gauss rule of the Boys
+// moments (rows: load_moment_rows), else the Chebyshev tables.
+template <int N>
+__device__ __forceinline__ void rys_roots(const JKRysTable &tab, const lds_double *rows,
+                                          double x, double *r, double *w)
 {
     if (x >= tab.xmax[N-1]) {
-        const double *lr = tab.coef + tab.large_r + N * (N - 1) / 2;
-        const double *lw = tab.coef + tab.large_w + N * (N - 1) / 2;
-        double ix = 1. / x;
-        double sx = sqrt(ix);
+        const double ix = rcp64(x), sx = rsqrt64(x);
+        if constexpr (N <= 3) {
+            constexpr double LR[6] = {0.5, 0.27525512860841095, 2.724744871391589,
+                                      0.19016350919348812, 1.7844927485432516, 5.52534374226326};
+            constexpr double LW[6] = {0.886226925452758, 0.8049140900055128, 0.08131283544724517,
+                                      0.7246295952243925, 0.15706732032285664,
+                                      0.004530009905508846};
 #pragma unroll
-        for (int i = 0; i < N; ++i) { r[i] = lr[i] * ix; w[i] = lw[i] * sx; }
+            for (int i = 0; i < N; ++i) {
+                r[i] = LR[N * (N - 1) / 2 + i] * ix;
+                w[i] = LW[N * (N - 1) / 2 + i] * sx;
+            }
+        } else {
+            const double *lr = tab.coef + tab.large_r + N * (N - 1) / 2;
+            const double *lw = tab.coef + tab.large_w + N * (N - 1) / 2;
+#pragma unroll
+            for (int i = 0; i < N; ++i) { r[i] = lr[i] * ix; w[i] = lw[i] * sx; }
+        }
         return;
     }
     if constexpr (N == 1) {
         double f[2];
-        boys_moments<2>(tab, x, f);
+        boys_moments<1>(rows, x, f);
         w[0] = f[0];
-        r[0] = f[1] / f[0];
+        r[0] = div64(f[1], f[0]);
         return;
     } else if constexpr (N == 2) {
         // monic p(u) = u^2 + c1 u + c0 orthogonal to 1 and u under the
         // moments: F2 + c1 F1 + c0 F0 = 0, F3 + c1 F2 + c0 F1 = 0
+        // (c1 < 0: both nodes are positive)
         double f[4];
-        boys_moments<4>(tab, x, f);
-        const double idet = 1. / (f[1] * f[1] - f[0] * f[2]);
+        boys_moments<2>(rows, x, f);
+        const double idet = rcp64(f[1] * f[1] - f[0] * f[2]);
         const double c1 = (f[0] * f[3] - f[1] * f[2]) * idet;
         const double c0 = (f[2] * f[2] - f[1] * f[3]) * idet;
-        const double disc = sqrt(c1 * c1 - 4. * c0);
-        const double q = -.5 * (c1 + copysign(disc, c1));
-        const double ua = q, ub = c0 / q;
-        const double u1 = fmin(ua, ub), u2 = fmax(ua, ub);
-        const double w1 = (f[1] - u2 * f[0]) / (u1 - u2);
+        const double disc = sqrt64(c1 * c1 - 4. * c0);
+        const double u2 = .5 * (disc - c1), u1 = div64(c0, u2);
+        const double w1 = div64(u2 * f[0] - f[1], u2 - u1);
         r[0] = u1; r[1] = u2;
         w[0] = w1; w[1] = f[0] - w1;
         return;
@@ -399,46 +492,48 @@ __device__ __forceinline__ void rys_roots(const JKRysTable &tab, double x,
         // recurrence coefficients of the monic orthogonal polynomials from
         // the moments (Chebyshev's algorithm, Gautschi 2004, Alg. 2.1), the
         // nodes from Viete's trigonometric solution of the characteristic
-        // cubic of the Jacobi matrix refined by two Newton steps on the
-        // three-term recurrence, the weights by the Christoffel formula
+        // cubic of the Jacobi matrix (in float: a starting point good to
+        // 1e-5) refined by two Newton steps on the three-term recurrence
+        // (1e-10, 1e-20), the weights by the Christoffel formula
         double mu[6];
-        boys_moments<6>(tab, x, mu);
-        const double a0 = mu[1] / mu[0], b0 = mu[0];
+        boys_moments<3>(rows, x, mu);
+        const double r0 = rcp64(mu[0]);
+        const double a0 = mu[1] * r0;
         const double n1 = mu[2] - a0 * mu[1], n2 = mu[3] - a0 * mu[2];
         const double n3 = mu[4] - a0 * mu[3], n4 = mu[5] - a0 * mu[4];
-        const double a1 = n2 / n1 - a0, b1 = n1 / mu[0];
+        const double rn1 = rcp64(n1);
+        const double q1 = n2 * rn1, a1 = q1 - a0, b1 = n1 * r0;
         const double m2 = n3 - a1 * n2 - b1 * mu[2], m3 = n4 - a1 * n3 - b1 * mu[3];
-        const double a2 = m3 / m2 - n2 / n1, b2 = m2 / n1;
+        const double rm2 = rcp64(m2);
+        const double a2 = m3 * rm2 - q1, b2 = m2 * rn1;
         const double c2 = -(a0 + a1 + a2);
         const double c1 = a0 * a1 + a0 * a2 + a1 * a2 - b1 - b2;
         const double c0 = b2 * a0 + b1 * a2 - a0 * a1 * a2;
         const double p = c1 - c2 * c2 * (1. / 3.);
         const double q = c2 * c2 * c2 * (2. / 27.) - c2 * c1 * (1. / 3.) + c0;
-        const double rr = sqrt(-p * (1. / 3.));
-        const double phi = acos(fmin(1., fmax(-1., -q / (2. * rr * rr * rr))));
-        double u[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            u[k] = 2. * rr * cos((phi - 2. * M_PI * k) * (1. / 3.)) - c2 * (1. / 3.);
-        const double nrm1 = b0 * b1, nrm2 = nrm1 * b2;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            double v = u[k];
+        const float rr = sqrtf((float)(-p) * (1.f / 3.f));
+        const float phi = acosf(fminf(1.f, fmaxf(-1.f, -(float)q / (2.f * rr * rr * rr))));
+        auto node = [&](float shift, double &rk, double &wk) {
+            double v = (double)(2.f * rr * __cosf((phi + shift) * (1.f / 3.f))) - c2 * (1. / 3.);
+            double p1, p2;
 #pragma unroll
             for (int it = 0; it < 2; ++it) {
-                const double p1 = v - a0;
-                const double p2 = (v - a1) * p1 - b1, d2 = p1 + (v - a1);
+                p1 = v - a0;
+                p2 = (v - a1) * p1 - b1;
+                const double d2 = p1 + (v - a1);
                 const double p3 = (v - a2) * p2 - b2 * p1, d3 = p2 + (v - a2) * d2 - b2;
-                v -= p3 / d3;
+                v -= p3 * __builtin_amdgcn_rcp(d3);
             }
-            const double p1 = v - a0, p2 = (v - a1) * p1 - b1;
-            w[k] = 1. / (1. / b0 + p1 * p1 / nrm1 + p2 * p2 / nrm2);
-            u[k] = v;
-        }
-        // ascending order (cos is decreasing on [0, pi]: k = 0 is the largest)
-        r[0] = u[2]; r[1] = u[1]; r[2] = u[0];
-        const double w0 = w[0];
-        w[0] = w[2]; w[2] = w0;
+            p1 = v - a0;
+            p2 = (v - a1) * p1 - b1;
+            // squared norms of the polynomials: mu_0, n1 = b0 b1, m2 = b0 b1 b2
+            wk = rcp64(r0 + p1 * p1 * rn1 + p2 * p2 * rm2);
+            rk = v;
+        };
+        // ascending: the node of phi + 2 pi is the smallest
+        node(2.f * (float)M_PI, r[0], w[0]);
+        node(-2.f * (float)M_PI, r[1], w[1]);
+        node(0.f, r[2], w[2]);
         return;
     }
     const int D1 = tab.degree + 1;
@@ -468,15 +563,6 @@ __device__ __forceinline__ void rys_root_one(const JKRysTable &tab, double x, in
         double ix = 1. / x;
         r = tab.coef[tab.large_r + N * (N - 1) / 2 + i] * ix;
         w = tab.coef[tab.large_w + N * (N - 1) / 2 + i] * sqrt(ix);
-        return;
-    }
-    if constexpr (N <= ROOT_ONE_BOYS_NMAX) {
-        double rr[N], ww[N];
-        rys_roots<N>(tab, x, rr, ww);
-        r = rr[0]; w = ww[0];
-#pragma unroll
-        for (int k = 1; k < N; ++k)
-            if (i == k) { r = rr[k]; w = ww[k]; }
         return;
     }
     const int D1 = tab.degree + 1;
@@ -891,7 +977,8 @@ __device__ __forceinline__ void krows_flush(const KRows &kr, int nfi, int nfj, i
 // Rys roots in FP32: Chebyshev series in float on the float copy of the
 // table; the large-x asymptotic branch is evaluated in FP64.
 template <int N>
-__device__ __forceinline__ void rys_roots(const JKRysTable &tab, float x, float *r, float *w)
+__device__ __forceinline__ void rys_roots(const JKRysTable &tab, const lds_double *, float x,
+                                          float *r, float *w)
 {
     if (x >= (float)tab.xmax[N-1]) {
         double xd = x;
@@ -930,7 +1017,8 @@ __device__ __forceinline__ void eri_lane(T *gout, const double *pij, int nij,
                                          const double *pkl, int nkl,
                                          const double *ri, const double *rij,
                                          const double *rk, const double *rkl,
-                                         const JKRysTable &rys, double fac_sym, double omega2)
+                                         const JKRysTable &rys, const lds_double *rows,
+                                         double fac_sym, double omega2)
 {
     constexpr int NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
     constexpr int NF = (I1 - I0) * NFJ * NFK * NFL;
@@ -961,23 +1049,23 @@ __device__ __forceinline__ void eri_lane(T *gout, const double *pij, int nij,
                 PQ[d] = (T)(p[2+d] - q[2+d]);
             }
             T rr = PQ[0]*PQ[0] + PQ[1]*PQ[1] + PQ[2]*PQ[2];
-            T r_aa = (T)1 / (aij + akl);
+            T r_aa = rcp64(aij + akl);
             T theta = aij * akl * r_aa;
-            T fac = (T)p[5] * Kkl * sqrt(r_aa);
+            T fac = (T)p[5] * Kkl * rsqrt64(aij + akl);
             T rt[N], wt[N];
             // long-range attenuation erf(omega r)/r: the rule at x a with the
             // roots scaled by a and the weights by sqrt(a)
             T aw = (T)1;
             if (omega2 > 0.) aw = (T)omega2 / ((T)omega2 + theta);
             if constexpr (sizeof(T) == sizeof(float) && N <= 3) {
-                // the Boys-grid rule in FP64 is cheaper than the float
+                // the rule of the Boys moments in FP64 is cheaper than the float
                 // Chebyshev series for up to three roots
                 double rd[N], wd[N];
-                rys_roots<N>(rys, (double)(theta * rr * aw), rd, wd);
+                rys_roots<N>(rys, rows, (double)(theta * rr * aw), rd, wd);
 #pragma unroll
                 for (int i = 0; i < N; ++i) { rt[i] = (T)rd[i]; wt[i] = (T)wd[i]; }
             } else {
-                rys_roots<N>(rys, theta * rr * aw, rt, wt);
+                rys_roots<N>(rys, rows, theta * rr * aw, rt, wt);
             }
             if (omega2 > 0.) {
                 const T sa = sqrt(aw);
@@ -1085,7 +1173,8 @@ __device__ __forceinline__ void lane_chunks(F &&f)
 template <int LI, int LJ, int LK, int LL, typename T>
 __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair &sp,
                                            uint32_t bas_ij, int pij, const uint32_t *queue,
-                                           int nb, int lane, uint64_t lt_mask, const KRows &kr)
+                                           int nb, int lane, uint64_t lt_mask, const KRows &kr,
+                                           const lds_double *rows)
 {
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
     constexpr int CH = LaneChunk<LI, LJ, LK, LL>::CH;
@@ -1127,7 +1216,7 @@ __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair
         T gout[NI * NFJ * NFK * NFL];
         eri_lane<LI, LJ, LK, LL, T, I0, I1>(gout, a.pdata_ij + (size_t)pij * nij * PREC, nij,
                                             a.pdata_kl + (size_t)pkl * nkl * PREC, nkl,
-                                            sp.ri, sp.rij, rk3, rkl, a.rys, fac_sym,
+                                            sp.ri, sp.rij, rk3, rkl, a.rys, rows, fac_sym,
                                             a.omega * a.omega);
         for (int id = 0; id < a.n_dm; ++id) {
             const double *D = a.dm + id * nao2;
@@ -1335,7 +1424,10 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     int kl_chunk, use_lds;
     const int item = select_task(a, batch, kl_chunk, use_lds);
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ);
+    constexpr int N = (LI + LJ + LK + LL) / 2 + 1;
     __shared__ uint32_t queue_all[LANE_WAVES][2][2 * WAVE];
+    __shared__ __align__(16) double moment_buf[MomentRows<N>::SIZE];
+    const lds_double *rows = (const lds_double *)moment_buf;
     const int lane = threadIdx.x & (WAVE - 1);
     const int wid = threadIdx.x / WAVE;
     uint32_t *queue64 = queue_all[wid][0];
@@ -1355,8 +1447,9 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     if (kr.on) {
         krows_zero(kr, NFI + NFJ, threadIdx.x, LANE_WAVES * WAVE);
         krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, LANE_WAVES * WAVE);
-        __syncthreads();
     }
+    load_moment_rows<N>(moment_buf, a.rys, threadIdx.x, LANE_WAVES * WAVE);
+    __syncthreads();
     int qn64 = 0, qn32 = 0;
     unsigned long long nsurv = 0, nsurv32 = 0, hsum = 0;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -1396,7 +1489,7 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
             const int nb = min(qn64, WAVE);
             if constexpr (PM != 2)
                 lane_batch<LI, LJ, LK, LL, double>(a, sp, bas_ij, wi.pij, queue64, nb, lane,
-                                                   lt_mask, kr);
+                                                   lt_mask, kr, rows);
             wave_sync();
             uint32_t rest = (nb + lane < qn64) ? queue64[nb + lane] : 0u;
             wave_sync();
@@ -1408,7 +1501,7 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
             const int nb = min(qn32, WAVE);
             if constexpr (PM != 1)
                 lane_batch<LI, LJ, LK, LL, float>(a, sp, bas_ij, wi.pij, queue32, nb, lane,
-                                                  lt_mask, kr);
+                                                  lt_mask, kr, rows);
             wave_sync();
             uint32_t rest = (nb + lane < qn32) ? queue32[nb + lane] : 0u;
             wave_sync();
@@ -1875,7 +1968,8 @@ static const ClassInfo *class_info()
             c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0>;
             c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1>;
             c.threads = LANE_WAVES * WAVE;
-            c.lds_static = sizeof(uint32_t) * LANE_WAVES * 2 * 2 * WAVE;
+            c.lds_static = sizeof(uint32_t) * LANE_WAVES * 2 * 2 * WAVE +
+                           sizeof(double) * MomentRows<T::N>::SIZE;
         } else {
             using S = TeamShape<LI, LJ, LK, LL>;
             c.fn[0] = c.fn[1] = (const void *)jk_team_kernel<LI, LJ, LK, LL>;

@@ -33,7 +33,8 @@ __device__ __forceinline__ void ip1_quartet(double *gi, double *gj, double *gk,
                                             const double *gamma, const JKBuildArgs &a,
                                             const ShellPair &sp, const double *pij, int nij,
                                             const double *pkl, int nkl, const double *rk,
-                                            const double *rkl, const double *expk, double omega2)
+                                            const double *rkl, const double *expk, double omega2,
+                                            const lds_double *rows)
 {
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
     constexpr int N = (LI + LJ + LK + LL + 1) / 2 + 1;
@@ -59,16 +60,16 @@ __device__ __forceinline__ void ip1_quartet(double *gi, double *gj, double *gk,
                 PQ[d] = p[2 + d] - q[2 + d];
             }
             const double rr = PQ[0]*PQ[0] + PQ[1]*PQ[1] + PQ[2]*PQ[2];
-            const double r_aa = 1. / (aij + akl);
+            const double r_aa = rcp64(aij + akl);
             const double theta = aij * akl * r_aa;
-            const double fac = p[5] * q[5] * sqrt(r_aa);
+            const double fac = p[5] * q[5] * rsqrt64(aij + akl);
             double aw = 1., sa = 1.;
             if (omega2 > 0.) {          // long-range attenuation (see eri_lane)
                 aw = omega2 / (omega2 + theta);
                 sa = sqrt(aw);
             }
             double rt[N], wt[N];
-            rys_roots<N>(a.rys, theta * rr * aw, rt, wt);
+            rys_roots<N>(a.rys, rows, theta * rr * aw, rt, wt);
             double ui[3] = {0., 0., 0.}, uj[3] = {0., 0., 0.}, uk[3] = {0., 0., 0.};
 #pragma unroll
             for (int r = 0; r < N; ++r) {
@@ -137,7 +138,10 @@ __global__ __launch_bounds__(WAVE)
 void jk_ip1_lane_kernel(JKBuildArgs a, TaskBatch batch, GenExtra ex)
 {
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
+    constexpr int N = (LI + LJ + LK + LL + 1) / 2 + 1;
     __shared__ uint32_t queue[2 * WAVE];
+    __shared__ __align__(16) double moment_buf[MomentRows<N>::SIZE];
+    const lds_double *rows = (const lds_double *)moment_buf;
     int kl_chunk, unused;
     const int item = select_task(a, batch, kl_chunk, unused);
     const int lane = threadIdx.x;
@@ -155,6 +159,8 @@ void jk_ip1_lane_kernel(JKBuildArgs a, TaskBatch batch, GenExtra ex)
     const double *pij = a.pdata_ij + (size_t)wi.pij * nij * PREC;
     const double omega2 = a.omega * a.omega;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    load_moment_rows<N>(moment_buf, a.rys, lane, WAVE);
+    __syncthreads();
     double gij[6];
 #pragma unroll
     for (int t = 0; t < 6; ++t) gij[t] = 0.;
@@ -261,7 +267,7 @@ void jk_ip1_lane_kernel(JKBuildArgs a, TaskBatch batch, GenExtra ex)
             double gi[3] = {0., 0., 0.}, gj[3] = {0., 0., 0.}, gk[3] = {0., 0., 0.};
             ip1_quartet<LI, LJ, LK, LL>(gi, gj, gk, gamma, a, sp, pij, nij,
                                         a.pdata_kl + (size_t)pkl * nkl * PREC, nkl, rk3, rkl,
-                                        a.env + a.bas[ksh * 8 + 5], omega2);
+                                        a.env + a.bas[ksh * 8 + 5], omega2, rows);
             if (active) {
                 double *ek = ex.ejk + 3 * a.bas[ksh * 8], *el = ex.ejk + 3 * a.bas[lsh * 8];
 #pragma unroll

@@ -267,6 +267,16 @@ static bool table_ok(const JKRysTable &t)
     return t.coef != nullptr && t.degree > 0 && t.degree <= RYS_DEG_MAX;
 }
 
+// whether the table holds the rule of n roots
+static bool table_has(const JKRysTable &t, int n)
+{
+    if (n > JK_RYS_NMAX || t.xmax[n-1] <= 0) return false;
+    // the moment rows as the kernels copy them
+    return n > 3 || (t.boys_rows == moment_rows(1) + moment_rows(2) + moment_rows(3) &&
+                     t.boys_step == MOMENT_STEP && t.boys % 2 == 0 &&
+                     t.xmax[n-1] <= (moment_rows(n) - .5) * MOMENT_STEP);
+}
+
 extern "C" {
 
 const char *jk_last_error(void) { return g_err; }
@@ -358,7 +368,7 @@ static int check_build(const JKBuildArgs *args, JKBuildArgs &a)
         return 3;
     }
     int nroots = (a.li + a.lj + a.lk + a.ll) / 2 + 1;
-    if (nroots > JK_RYS_NMAX || a.rys.xmax[nroots-1] <= 0) {
+    if (!table_has(a.rys, nroots)) {
         set_err("jk_build: Rys table lacks %d roots", nroots);
         return 3;
     }
@@ -379,7 +389,7 @@ static int check_ip1(const JKBuildArgs *args, JKBuildArgs &a, const double *ejk)
         return 3;
     }
     const int nroots = (a.li + a.lj + a.lk + a.ll + 1) / 2 + 1;
-    if (nroots > JK_RYS_NMAX || a.rys.xmax[nroots-1] <= 0) {
+    if (!table_has(a.rys, nroots)) {
         set_err("jk_energy_ip1: Rys table lacks %d roots", nroots);
         return 3;
     }

@@ -14,9 +14,9 @@ _here = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_here, 'libjkhip.so')
 TABLE_PATH = os.path.join(os.path.dirname(_here), 'csrc', 'rys_table.npz')
 
-JK_ABI_VERSION = 13
+JK_ABI_VERSION = 14
 JK_RYS_NMAX = 11
-JK_BOYS_M = 13
+JK_BOYS_M = 14
 JK_LMAX = 5
 # JKBuildArgs.screen
 JK_SCREEN = {'jk': 0, 'j': 1, 'k': 2}
@@ -186,13 +186,15 @@ def load_rys_table_host():
     coef = t['coef']
     lr = t['large_r']
     lw = t['large_w']
-    boys = np.ascontiguousarray(t['boys'], dtype=np.float64)
-    assert boys.shape[1] == JK_BOYS_M
-    data = np.concatenate([coef, lr, lw, boys.ravel()]).astype(np.float64)
+    rows = [np.ascontiguousarray(t[f'moments{n}'], dtype=np.float64) for n in (1, 2, 3)]
+    assert all(r.shape[1] == JK_BOYS_M for r in rows)
+    head = np.concatenate([coef, lr, lw])
+    head = np.concatenate([head, np.zeros(len(head) % 2)])      # 16-byte aligned rows
+    data = np.concatenate([head] + [r.ravel() for r in rows]).astype(np.float64)
     meta = dict(off=t['off'].astype(np.int64), xmax=t['xmax'].astype(np.float64),
                 large_r=len(coef), large_w=len(coef) + len(lr), degree=int(t['degree']),
-                boys=len(coef) + len(lr) + len(lw), boys_rows=boys.shape[0],
-                boys_step=float(t['boys_step']))
+                boys=len(head), boys_rows=sum(len(r) for r in rows),
+                boys_step=float(t['moment_step']))
     return data, meta
 
 

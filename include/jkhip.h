@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define JK_ABI_VERSION  13
+#define JK_ABI_VERSION  14
 #define JK_RYS_NMAX     11      /* max Rys roots: (hh|hh) */
 #define JK_LMAX         5       /* max angular momentum on the GPU path */
 
@@ -32,9 +32,11 @@ extern "C" {
  * coef[off[n-1] + (k*2n + f)*(degree+1) + d] on unit intervals [k, k+1),
  * k < xmax[n-1]; above, u_i = large[n*(n-1)/2 + i] / x and
  * w_i = large[large_w + n*(n-1)/2 + i] / sqrt(x).
- * Boys grid (one to three roots): coef[boys + g*JK_BOYS_M + m] = F_m(g*boys_step),
- * boys_rows grid points covering x < xmax[2]. */
-#define JK_BOYS_M       13
+ * Moment rows (rules of n = 1, 2, 3 roots): 79, 95 and 109 rows (boys_rows in
+ * all) of JK_BOYS_M doubles each, the rows of n after those of n - 1, from
+ * coef[boys] on, 16-byte aligned; row g holds F_{2n-1+k}(x_g) / k! for k < 12, exp(-x_g) and 0 for
+ * x_g = g * boys_step (0.5), covering x < xmax[n-1]. */
+#define JK_BOYS_M       14
 typedef struct {
     const double *coef;
     const float *coef32;        /* coef rounded to float (FP32 quartets) */
@@ -44,7 +46,7 @@ typedef struct {
     int64_t large_w;            /* offset of large-x weights in coef */
     int degree;
     int boys_rows;
-    int64_t boys;               /* offset of the Boys grid in coef */
+    int64_t boys;               /* offset of the moment rows in coef */
     double boys_step, boys_inv_step;
 } JKRysTable;
 
