@@ -70,11 +70,6 @@
 #ifndef LANE_SKIP_NF
 #define LANE_SKIP_NF    0
 #endif
-// wavefronts per block of the per-lane kernel (32-water def2-TZVP build on
-// three streams, ms: 1 -> 546, 2 -> 464, 4 -> 489)
-#ifndef LANE_WAVES
-#define LANE_WAVES      2
-#endif
 // launch shapes: work items of the per-lane kernel target LANE_ITEMS blocks
 // per launch with at least LANE_MIN_CHUNK kl candidates each; the team
 // kernel scans TEAM_KL_CHUNK candidates per work item.  Measured on the
@@ -775,6 +770,32 @@ __device__ __forceinline__ bool survives_dmax(float q_kl, float kl_cutoff, float
     return dmax > d_cutoff;
 }
 
+// Same predicate with the shells of kl and dm_cond[bas_ij] at hand.
+__device__ __forceinline__ bool survives_sh(float q_kl, float kl_cutoff, float dm_penalty,
+                                            uint32_t bas_ij, uint32_t bas_kl, int ish, int jsh,
+                                            int ksh, int lsh, int nbas, const float *dm_cond,
+                                            float dc_ij, int screen, bool swapped, float q_ij,
+                                            float cutoff)
+{
+    if (swapped) {
+        kl_cutoff = cutoff - q_kl;
+        q_kl = q_ij;
+    }
+    if (!(q_kl + dm_penalty >= kl_cutoff && (swapped ? bas_kl >= bas_ij : bas_ij >= bas_kl)))
+        return false;
+    const float d_cutoff = kl_cutoff - q_kl;
+    float dmax = -1e30f;
+    if (screen != JK_SCREEN_K) dmax = fmaxf(dc_ij, dm_cond[bas_kl]);
+    // the exchange blocks D_ik, D_jk, D_il, D_jl of the task's shells
+    if (screen != JK_SCREEN_J) {
+        const int s1 = swapped ? nbas : 1, sk = swapped ? 1 : nbas;
+        const float *di = dm_cond + ish * sk, *dj = dm_cond + jsh * sk;
+        dmax = fmaxf(dmax, fmaxf(fmaxf(di[ksh * s1], dj[ksh * s1]),
+                                 fmaxf(di[lsh * s1], dj[lsh * s1])));
+    }
+    return dmax > d_cutoff;
+}
+
 // Work item of a launch: pair_ij index and the kl range of its chunk.
 // One work item: ij pair pij against kl pairs [kl0, kl1), whose k and l AOs
 // lie in [k_ao0, k_ao0 + k_nao) and [l_ao0, l_ao0 + l_nao) (the K-row
@@ -1008,17 +1029,58 @@ __device__ __forceinline__ void rys_roots(const JKRysTable &tab, const lds_doubl
     }
 }
 
+// The primitives of the (uniform) ij pair: a, 1/a, P, K, P - R_i of record ip,
+// from the pair records in HBM or from their copy in LDS (stage_pij).
+#define PIJ_LDS 10      // doubles of one primitive's copy
+struct PijGlobal {
+    const double *rec, *ri;
+    __device__ __forceinline__ void get(int ip, double &a, double &ra, double *P, double &K,
+                                        double *PA) const
+    {
+        const double *p = rec + ip * PREC;
+        a = p[0]; ra = p[1]; K = p[5];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { P[d] = p[2+d]; PA[d] = p[2+d] - ri[d]; }
+    }
+};
+
+struct PijLds {
+    const lds_double *rec;
+    __device__ __forceinline__ void get(int ip, double &a, double &ra, double *P, double &K,
+                                        double *PA) const
+    {
+        const lds_double2 *p = (const lds_double2 *)(rec + ip * PIJ_LDS);
+        const double2v v0 = p[0], v1 = p[1], v2 = p[2], v3 = p[3], v4 = p[4];
+        a = v0.x; ra = v0.y;
+        P[0] = v1.x; P[1] = v1.y; P[2] = v2.x; K = v2.y;
+        PA[0] = v3.x; PA[1] = v3.y; PA[2] = v4.x;
+    }
+};
+
+// copies the records of the work item's ij pair (a barrier must follow)
+__device__ __forceinline__ void stage_pij(lds_double *dst, const double *rec, int nij,
+                                          const double *ri, int tid, int nthreads)
+{
+    for (int n = tid; n < nij; n += nthreads) {
+        const double *p = rec + n * PREC;
+        lds_double *o = dst + n * PIJ_LDS;
+        o[0] = p[0]; o[1] = p[1]; o[2] = p[2]; o[3] = p[3]; o[4] = p[4]; o[5] = p[5];
+        o[6] = p[2] - ri[0]; o[7] = p[3] - ri[1]; o[8] = p[4] - ri[2];
+    }
+}
+
 // One quartet per lane in arithmetic type T (double or float): returns the
 // rows I0 <= i < I1 of the Cartesian block (times the symmetry and
 // normalisation prefactors) in gout[(((i-I0)*nfj+j)*nfk+k)*nfl+l].
-// pij: records of the (uniform) ij pair; pkl: records of this lane's kl pair.
-template <int LI, int LJ, int LK, int LL, typename T, int I0 = 0, int I1 = ncart(LI)>
-__device__ __forceinline__ void eri_lane(T *gout, const double *pij, int nij,
-                                         const double *pkl, int nkl,
-                                         const double *ri, const double *rij,
+// pij: the primitives of the (uniform) ij pair; pkl: records of this lane's kl
+// pair.  `loaded` is called once, when the first kl record has arrived.
+template <int LI, int LJ, int LK, int LL, typename T, int I0 = 0, int I1 = ncart(LI),
+          typename Pij, typename F>
+__device__ __forceinline__ void eri_lane(T *gout, const Pij &pij, int nij,
+                                         const double *pkl, int nkl, const double *rij,
                                          const double *rk, const double *rkl,
                                          const JKRysTable &rys, const lds_double *rows,
-                                         double fac_sym, double omega2)
+                                         double fac_sym, double omega2, F &&loaded)
 {
     constexpr int NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
     constexpr int NF = (I1 - I0) * NFJ * NFK * NFL;
@@ -1032,26 +1094,34 @@ __device__ __forceinline__ void eri_lane(T *gout, const double *pij, int nij,
     const T rkl_t[3] = {(T)rkl[0], (T)rkl[1], (T)rkl[2]};
 #pragma unroll
     for (int n = 0; n < NF; ++n) gout[n] = 0;
+    double q[PREC];
+#pragma unroll
+    for (int n = 0; n < PREC; ++n) q[n] = pkl[n];
+    loaded();
     for (int kp = 0; kp < nkl; ++kp) {
-        const double *q = pkl + kp * PREC;
+        if (kp > 0) {
+#pragma unroll
+            for (int n = 0; n < PREC; ++n) q[n] = pkl[kp * PREC + n];
+        }
         const T akl = (T)q[0], rakl = (T)q[1];
         const T Kkl = (T)(q[5] * fac_sym);
         T QC[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) QC[d] = (T)(q[2+d] - rk[d]);
         for (int ip = 0; ip < nij; ++ip) {
-            const double *p = pij + ip * PREC;
-            const T aij = (T)p[0], raij = (T)p[1];
+            double a_d, ra_d, P_d[3], K_d, PA_d[3];
+            pij.get(ip, a_d, ra_d, P_d, K_d, PA_d);
+            const T aij = (T)a_d, raij = (T)ra_d;
             T PA[3], PQ[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                PA[d] = (T)(p[2+d] - ri[d]);
-                PQ[d] = (T)(p[2+d] - q[2+d]);
+                PA[d] = (T)PA_d[d];
+                PQ[d] = (T)(P_d[d] - q[2+d]);
             }
             T rr = PQ[0]*PQ[0] + PQ[1]*PQ[1] + PQ[2]*PQ[2];
             T r_aa = rcp64(aij + akl);
             T theta = aij * akl * r_aa;
-            T fac = (T)p[5] * Kkl * rsqrt64(aij + akl);
+            T fac = (T)K_d * Kkl * rsqrt64(aij + akl);
             T rt[N], wt[N];
             // long-range attenuation erf(omega r)/r: the rule at x a with the
             // roots scaled by a and the weights by sqrt(a)
@@ -1214,10 +1284,10 @@ __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair
         constexpr int I1 = I0 + CH < NFI ? I0 + CH : NFI;
         constexpr int NI = I1 - I0;
         T gout[NI * NFJ * NFK * NFL];
-        eri_lane<LI, LJ, LK, LL, T, I0, I1>(gout, a.pdata_ij + (size_t)pij * nij * PREC, nij,
-                                            a.pdata_kl + (size_t)pkl * nkl * PREC, nkl,
-                                            sp.ri, sp.rij, rk3, rkl, a.rys, rows, fac_sym,
-                                            a.omega * a.omega);
+        eri_lane<LI, LJ, LK, LL, T, I0, I1>(
+            gout, PijGlobal{a.pdata_ij + (size_t)pij * nij * PREC, sp.ri}, nij,
+            a.pdata_kl + (size_t)pkl * nkl * PREC, nkl, sp.rij, rk3, rkl, a.rys, rows, fac_sym,
+            a.omega * a.omega, [] {});
         for (int id = 0; id < a.n_dm; ++id) {
             const double *D = a.dm + id * nao2;
             if (a.vk) {
@@ -1386,8 +1456,8 @@ __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair
     });
 }
 
-// Per-lane kernel.  LANE_WAVES wavefronts share one work item (and its LDS K
-// rows); each wavefront scans every LANE_WAVES-th batch of 64 kl candidates
+// Per-lane kernel.  NW wavefronts share one work item (and its LDS K
+// rows); each wavefront scans every NW-th batch of 64 kl candidates
 // and keeps two queues: quartets whose bound q_ij + q_kl + max(dm_cond)
 // reaches fp32_cut run in FP64, the others in FP32.  PM (precision mode):
 // 0 both queues, 1 the FP64 queue only, 2 the FP32 queue only (a launch
@@ -1396,6 +1466,24 @@ __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair
 // (64-water build 2110 -> 2092 ms against PM 0); mixed builds PM 0, since
 // the pair PM 1 + PM 2 scans and flushes every work item twice (2115 ->
 // 2253 ms; the FP32-only kernels mostly keep the occupancy of PM 0).
+// Wavefronts per workgroup of the per-lane kernels.  The K and density rows of a
+// work item are LDS that its wavefronts share: four of them where the registers
+// leave room for more wavefronts than the rows of two-wave workgroups do.
+// 48 waters (def2-TZVP), one stream, ms, two waves -> four: (ps|ss) 58.5 -> 50.7,
+// (fs|ps) 37.3 -> 31.4, (ff|ps) 24.9 -> 19.5, (ds|ss) 24.5 -> 19.1, (fs|ss)
+// 20.9 -> 16.1, (pp|ss) 19.9 -> 14.7, (fp|ss) 19.4 -> 17.2, (ff|ss) 16.4 -> 12.1,
+// (dp|ss) 13.7 -> 9.7; slower the classes at one wave per SIMD ((fp|ps)
+// 30.6 -> 34.0, (dp|ps) 34.3 -> 38.0, (fs|ds) 22.7 -> 27.1, (pp|pp) 12.4 -> 14.6).
+// Eight: the whole build 1103 -> 1230 ((ff|ps) 19.3 -> 53.6, (ps|ps) 57 -> 64).
+template <int LI, int LJ, int LK, int LL> struct FourWaves { static constexpr bool ON = false; };
+#define LANE_WAVES4(a, b, c, d) \
+    template <> struct FourWaves<a, b, c, d> { static constexpr bool ON = true; };
+LANE_WAVES4(1, 0, 0, 0) LANE_WAVES4(1, 0, 1, 0) LANE_WAVES4(1, 1, 0, 0) LANE_WAVES4(1, 1, 1, 0)
+LANE_WAVES4(2, 0, 0, 0) LANE_WAVES4(2, 0, 1, 0) LANE_WAVES4(2, 0, 1, 1) LANE_WAVES4(2, 0, 2, 0)
+LANE_WAVES4(2, 1, 0, 0) LANE_WAVES4(2, 2, 0, 0) LANE_WAVES4(3, 0, 0, 0) LANE_WAVES4(3, 0, 1, 0)
+LANE_WAVES4(3, 1, 0, 0) LANE_WAVES4(3, 2, 1, 0) LANE_WAVES4(3, 3, 0, 0) LANE_WAVES4(3, 3, 1, 0)
+#undef LANE_WAVES4
+
 // Minimum waves per SIMD a class kernel is compiled for.  By default the
 // compiler may use all 512 registers (one wave per SIMD); the classes below
 // need a little over 256 and run faster with two waves per SIMD despite a few
@@ -1417,15 +1505,15 @@ CLASS_OCC2(3, 2, 3, 0)
 #undef CLASS_OCC2
 
 
-template <int LI, int LJ, int LK, int LL, int PM>
-__global__ __launch_bounds__(LANE_WAVES * WAVE, (ClassOcc<LI, LJ, LK, LL>::W))
+template <int LI, int LJ, int LK, int LL, int PM, int NW>
+__global__ __launch_bounds__((NW * WAVE), (ClassOcc<LI, LJ, LK, LL>::W))
 void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
 {
     int kl_chunk, use_lds;
     const int item = select_task(a, batch, kl_chunk, use_lds);
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ);
     constexpr int N = (LI + LJ + LK + LL) / 2 + 1;
-    __shared__ uint32_t queue_all[LANE_WAVES][2][2 * WAVE];
+    __shared__ uint32_t queue_all[NW][2][2 * WAVE];
     __shared__ __align__(16) double moment_buf[MomentRows<N>::SIZE];
     const lds_double *rows = (const lds_double *)moment_buf;
     const int lane = threadIdx.x & (WAVE - 1);
@@ -1445,17 +1533,17 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     extern __shared__ double kacc_dyn[];
     const KRows kr = make_krows(kacc_dyn, use_lds, NFI + NFJ, wi);
     if (kr.on) {
-        krows_zero(kr, NFI + NFJ, threadIdx.x, LANE_WAVES * WAVE);
-        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, LANE_WAVES * WAVE);
+        krows_zero(kr, NFI + NFJ, threadIdx.x, NW * WAVE);
+        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, NW * WAVE);
     }
-    load_moment_rows<N>(moment_buf, a.rys, threadIdx.x, LANE_WAVES * WAVE);
+    load_moment_rows<N>(moment_buf, a.rys, threadIdx.x, NW * WAVE);
     __syncthreads();
     int qn64 = 0, qn32 = 0;
     unsigned long long nsurv = 0, nsurv32 = 0, hsum = 0;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     bool stop = false;
     for (int base = wi.kl0 + wid * WAVE; base < wi.kl1 || qn64 > 0 || qn32 > 0;
-         base += LANE_WAVES * WAVE) {
+         base += NW * WAVE) {
         if (base < wi.kl1 && !stop) {
             int pkl = base + lane;
             bool keep = false, fail_margin = false, lowp = false;
@@ -1484,7 +1572,7 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
             stop = __ballot(fail_margin) != 0;
             wave_sync();
         }
-        const bool flush = (base + LANE_WAVES * WAVE >= wi.kl1) || stop;
+        const bool flush = (base + NW * WAVE >= wi.kl1) || stop;
         if (PM != 2 && (qn64 >= WAVE || (flush && qn64 > 0))) {
             const int nb = min(qn64, WAVE);
             if constexpr (PM != 2)
@@ -1513,12 +1601,307 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     }
     if (kr.on) {
         __syncthreads();
-        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, LANE_WAVES * WAVE);
+        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, NW * WAVE);
     }
     if (lane == 0) {
         if (a.n_quartets && nsurv) atomicAdd(a.n_quartets, nsurv);
         if (a.n_quartets_fp32 && nsurv32) atomicAdd(a.n_quartets_fp32, nsurv32);
     }
+    if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
+}
+
+// ---------------------------------------------------------------- one density
+// Per-lane kernel of the FP64 builds of one density with J and K (WJ, WK), J
+// only or K only: what jk_lane_kernel decides at run time -- which matrices,
+// where K is accumulated, the number of densities -- is fixed here, with the K
+// rows and the density rows of the work item in LDS (KR_DROWS), J_ij and D_ij
+// of the item in LDS, and its primitive records in LDS.
+// These kernels wait for memory more than they compute: the load counter of a
+// wavefront drains in order, so a load issued after the J_kl atomics of a batch
+// waits for them.  A batch therefore keeps its J_kl block in registers, and the
+// next batch adds it once its own first loads have arrived; the primitive loop
+// then reads LDS only (for a ket of one primitive pair).
+// 48 waters (def2-TZVP), one stream, ms: (ps|ss) 65.8 -> 58.5,
+// (dp|ps) 40.6 -> 34.3, (dp|ss) 17.0 -> 13.7, (ds|ss) 29.0 -> 24.5, (ds|ps) 38.9 -> 35.4;
+// the whole build on four streams 1000 -> 952.
+// Chunked classes with an f shell stay on jk_lane_kernel: the J_kl block held
+// over the chunks costs them more registers than the waits ((fp|fs) 20.8 -> 22.5,
+// (fp|pp) 33.7 -> 34.5, (fp|ds) 29.4 -> 29.9).
+template <int LI, int LJ, int LK, int LL>
+struct LaneFast {
+    static constexpr bool ON = LI < 3 || LaneChunk<LI, LJ, LK, LL>::NCH == 1;
+};
+
+struct ItemLds {
+    const lds_double *pij, *dij;
+    lds_double *jij;
+    const lds_double *rows;
+};
+
+template <int LI, int LJ, int LK, int LL, bool WJ, bool WK>
+__device__ __forceinline__ void lane_batch_fast(const JKBuildArgs &a, const ShellPair &sp,
+                                                int pkl, uint32_t sh, bool active, int lane,
+                                                const KRows &kr, const ItemLds &it,
+                                                double *pend, uint32_t &pend_off)
+{
+    constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
+    constexpr int CH = LaneChunk<LI, LJ, LK, LL>::CH;
+    const int nao = a.nao;
+    const int ksh = sh >> 16, lsh = sh & 0xffff;
+    double fac_sym = a.scale;
+    if (sp.ish == sp.jsh) fac_sym *= .5;
+    if (ksh == lsh) fac_sym *= .5;
+    if (sp.ish == ksh && sp.jsh == lsh) fac_sym *= .5;
+    if (!active) fac_sym = 0.;
+    const double *rk = a.env + a.bas[ksh * 8 + 7], *rl = a.env + a.bas[lsh * 8 + 7];
+    const double rk3[3] = {rk[0], rk[1], rk[2]};
+    const double rkl[3] = {rl[0] - rk[0], rl[1] - rk[1], rl[2] - rk[2]};
+    const int nij = a.iprim * a.jprim, nkl = a.kprim * a.lprim;
+    const int k0 = a.ao_loc[ksh], l0 = a.ao_loc[lsh];
+    // columns of this quartet's k and l AOs in the LDS rows
+    const int dk = k0 - kr.k_ao0, dl = kr.loff + l0 - kr.l_ao0;
+    const uint32_t off_kl = (uint32_t)k0 * (uint32_t)nao + (uint32_t)l0;
+    double vkl[NFK * NFL];
+#pragma unroll
+    for (int n = 0; n < NFK * NFL; ++n) vkl[n] = 0.;
+    lane_chunks<(NFI + CH - 1) / CH>([&](auto cc) {
+        constexpr int I0 = decltype(cc)::value * CH;
+        constexpr int I1 = I0 + CH < NFI ? I0 + CH : NFI;
+        constexpr int NI = I1 - I0;
+        double gout[NI * NFJ * NFK * NFL];
+        eri_lane<LI, LJ, LK, LL, double, I0, I1>(
+            gout, PijLds{it.pij}, nij, a.pdata_kl + (size_t)pkl * nkl * PREC, nkl, sp.rij, rk3,
+            rkl, a.rys, it.rows, fac_sym, a.omega * a.omega, [&] {
+                if constexpr (WJ && I0 == 0) {
+                    // J_kl of the previous batch
+                    if (pend_off != ~0u) {
+                        double *J = a.vj + pend_off;
+#pragma unroll
+                        for (int n = 0; n < NFK * NFL; ++n)
+                            atomic_add(J + (uint32_t)((n / NFL) * nao + n % NFL), pend[n]);
+                    }
+                }
+            });
+        if constexpr (WK) {
+            // K_ik += (ij|kl) D_jl ; K_il += (ij|kl) D_jk
+#pragma unroll
+            for (int i = I0; i < I1; ++i) {
+                double kil[NFL], kik[NFK];
+#pragma unroll
+                for (int l = 0; l < NFL; ++l) kil[l] = 0.;
+#pragma unroll
+                for (int k = 0; k < NFK; ++k) kik[k] = 0.;
+                if (active) {
+#pragma unroll
+                    for (int j = 0; j < NFJ; ++j) {
+                        const lds_double *dj = kr.d + (NFI + j) * kr.width;
+#pragma unroll
+                        for (int k = 0; k < NFK; ++k)
+#pragma unroll
+                        for (int l = 0; l < NFL; ++l) {
+                            const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
+                            kil[l] = fma(g, dj[dk + k], kil[l]);
+                            kik[k] = fma(g, dj[dl + l], kik[k]);
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < NFK; ++k) lds_add(kr.p + i * kr.width + dk + k, kik[k]);
+#pragma unroll
+                    for (int l = 0; l < NFL; ++l) lds_add(kr.p + i * kr.width + dl + l, kil[l]);
+                }
+            }
+            // K_jk += (ij|kl) D_il ; K_jl += (ij|kl) D_ik
+#pragma unroll
+            for (int j = 0; j < NFJ; ++j) {
+                double kjl[NFL], kjk[NFK];
+#pragma unroll
+                for (int l = 0; l < NFL; ++l) kjl[l] = 0.;
+#pragma unroll
+                for (int k = 0; k < NFK; ++k) kjk[k] = 0.;
+                if (active) {
+#pragma unroll
+                    for (int i = I0; i < I1; ++i) {
+                        const lds_double *di = kr.d + i * kr.width;
+#pragma unroll
+                        for (int k = 0; k < NFK; ++k)
+#pragma unroll
+                        for (int l = 0; l < NFL; ++l) {
+                            const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
+                            kjl[l] = fma(g, di[dk + k], kjl[l]);
+                            kjk[k] = fma(g, di[dl + l], kjk[k]);
+                        }
+                    }
+                    lds_double *kj = kr.p + (NFI + j) * kr.width;
+#pragma unroll
+                    for (int k = 0; k < NFK; ++k) lds_add(kj + dk + k, kjk[k]);
+#pragma unroll
+                    for (int l = 0; l < NFL; ++l) lds_add(kj + dl + l, kjl[l]);
+                }
+            }
+        }
+        if constexpr (WJ) {
+            double dkl[NFK * NFL];
+            const double *D = a.dm + off_kl;
+#pragma unroll
+            for (int n = 0; n < NFK * NFL; ++n) dkl[n] = D[(uint32_t)((n / NFL) * nao + n % NFL)];
+            double vij[NI * NFJ];
+#pragma unroll
+            for (int i = I0; i < I1; ++i)
+#pragma unroll
+            for (int j = 0; j < NFJ; ++j) {
+                const double d = it.dij[i * NFJ + j];
+                double s = 0.;
+#pragma unroll
+                for (int n = 0; n < NFK * NFL; ++n) {
+                    const double g = gout[((i - I0)*NFJ + j)*NFK*NFL + n];
+                    s = fma(g, dkl[n], s);
+                    vkl[n] = fma(g, d, vkl[n]);
+                }
+                // (an inactive lane's integrals are zero)
+                vij[(i - I0)*NFJ + j] = s;
+            }
+            wave_reduce_scatter<NI * NFJ>(vij, lane, [&](int n, double x) {
+                lds_add(it.jij + I0 * NFJ + n, x);
+            });
+        }
+    });
+    if constexpr (WJ) {
+#pragma unroll
+        for (int n = 0; n < NFK * NFL; ++n) pend[n] = vkl[n];
+        pend_off = active ? off_kl : ~0u;
+    }
+}
+
+template <int LI, int LJ, int LK, int LL, bool WJ, bool WK, int NW>
+__global__ __launch_bounds__((NW * WAVE), (ClassOcc<LI, LJ, LK, LL>::W))
+void jk_lane_fast_kernel(JKBuildArgs a, TaskBatch batch)
+{
+    int kl_chunk, use_lds;
+    const int item = select_task(a, batch, kl_chunk, use_lds);
+    constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFKL = ncart(LK) * ncart(LL);
+    constexpr int N = (LI + LJ + LK + LL) / 2 + 1;
+    constexpr int NT = NW * WAVE;
+    __shared__ uint32_t queue_all[NW][2][2 * WAVE];
+    __shared__ int left[NW];
+    __shared__ __align__(16) double moment_buf[MomentRows<N>::SIZE];
+    __shared__ double ij_buf[2][NFI * NFJ];
+    extern __shared__ __align__(16) double fast_dyn[];
+    const int tid = threadIdx.x;
+    const int lane = tid & (WAVE - 1);
+    const int wid = tid / WAVE;
+    uint32_t *queue = queue_all[wid][0], *queue_sh = queue_all[wid][1];
+    const int nbas = a.nbas, nao = a.nao;
+    select_replica(a);
+    const WorkItem wi = work_item(a, item, kl_chunk, use_lds);
+    const uint32_t bas_ij = a.pairs_ij[wi.pij];
+    const float q_ij = a.q_ij[wi.pij];
+    const float kl_cutoff = a.cutoff - q_ij;
+    if (a.q_kl[wi.kl0] + a.dm_penalty + Q_COND_MARGIN < kl_cutoff) return;
+    ShellPair sp;
+    load_shell_pair(sp, bas_ij, nbas, a.bas, a.env, a.ao_loc);
+    const float dc_ij = a.dm_cond[bas_ij];
+    const int nij = a.iprim * a.jprim;
+    // LDS: primitive records of ij, then the K rows and the density rows
+    ItemLds it;
+    lds_double *pij = (lds_double *)fast_dyn;
+    it.pij = pij;
+    it.dij = (lds_double *)ij_buf[0];
+    it.jij = (lds_double *)ij_buf[1];
+    it.rows = (lds_double *)moment_buf;
+    const KRows kr = make_krows(fast_dyn + nij * PIJ_LDS, WK ? 2 | KR_DROWS : 0, NFI + NFJ, wi);
+    if constexpr (WK) {
+        krows_zero(kr, NFI + NFJ, tid, NT);
+        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, tid, NT);
+    }
+    stage_pij(pij, a.pdata_ij + (size_t)wi.pij * nij * PREC, nij, sp.ri, tid, NT);
+    load_moment_rows<N>(moment_buf, a.rys, tid, NT);
+    for (int n = tid; n < NFI * NFJ; n += NT) {
+        ij_buf[0][n] = a.dm[(size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ];
+        ij_buf[1][n] = 0.;
+    }
+    __syncthreads();
+    int qn = 0;
+    unsigned long long nsurv = 0, hsum = 0;
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    double pend[WJ ? NFKL : 1];
+    uint32_t pend_off = ~0u;
+#pragma unroll
+    for (int n = 0; n < (WJ ? NFKL : 1); ++n) pend[n] = 0.;
+    // floor(b / nbas) of a pair id: the reciprocal's estimate is at most one
+    // too large
+    const uint32_t nbas_inv = 0xffffffffu / (uint32_t)nbas + 1u;
+    bool stop = false;
+    int base = wi.kl0 + wid * WAVE;
+    bool last = false;
+    while (!last) {
+        // survivors until a batch is full
+        while (qn < WAVE && base < wi.kl1 && !stop) {
+            const int pkl = base + lane;
+            bool keep = false, fail_margin = false;
+            uint32_t sh = 0;
+            if (pkl < wi.kl1) {
+                const float q_kl = a.q_kl[pkl];
+                const uint32_t bkl = a.pairs_kl[pkl];
+                fail_margin = q_kl + a.dm_penalty + Q_COND_MARGIN < kl_cutoff;
+                uint32_t ksh = nbas > 1 ? __umulhi(bkl, nbas_inv) : bkl;
+                if (ksh * (uint32_t)nbas > bkl) --ksh;
+                const uint32_t lsh = bkl - ksh * (uint32_t)nbas;
+                sh = ksh << 16 | lsh;
+                keep = survives_sh(q_kl, kl_cutoff, a.dm_penalty, bas_ij, bkl, sp.ish, sp.jsh,
+                                   (int)ksh, (int)lsh, nbas, a.dm_cond, dc_ij, a.screen,
+                                   a.swap_ijkl != 0, q_ij, a.cutoff);
+                if (a.quartet_hash && keep) hsum += task_mix(a, bas_ij, bkl);
+            }
+            const uint64_t m = __ballot(keep);
+            if (keep) {
+                const int n = qn + __popcll(m & lt_mask);
+                queue[n] = pkl;
+                queue_sh[n] = sh;
+            }
+            qn += __popcll(m);
+            nsurv += __popcll(m);
+            stop = __ballot(fail_margin) != 0;
+            wave_sync();
+            base += NT;
+        }
+        // the newest WAVE entries of the queue; at the end the wavefronts'
+        // remainders together, one batch each
+        int w = wid, n = qn - WAVE + lane;
+        bool active = true;
+        if (qn >= WAVE) {
+            qn -= WAVE;
+        } else {
+            if (lane == 0) left[wid] = qn;
+            __syncthreads();
+            int total = 0;
+#pragma unroll
+            for (int v = 0; v < NW; ++v) total += left[v];
+            if (wid * WAVE >= total) break;
+            active = wid * WAVE + lane < total;
+            n = active ? wid * WAVE + lane : 0;
+            for (w = 0; n >= left[w]; ++w) n -= left[w];
+            last = true;
+        }
+        lane_batch_fast<LI, LJ, LK, LL, WJ, WK>(a, sp, queue_all[w][0][n], queue_all[w][1][n],
+                                                active, lane, kr, it, pend, pend_off);
+        wave_sync();
+    }
+    if constexpr (WJ) {
+        if (pend_off != ~0u) {
+            constexpr int NFL = ncart(LL);
+            double *J = a.vj + pend_off;
+#pragma unroll
+            for (int n = 0; n < NFKL; ++n)
+                atomic_add(J + (uint32_t)((n / NFL) * nao + n % NFL), pend[n]);
+        }
+    }
+    __syncthreads();
+    if constexpr (WK) krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, tid, NT);
+    if constexpr (WJ) {
+        for (int n = tid; n < NFI * NFJ; n += NT)
+            atomic_add(a.vj + (size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ, ij_buf[1][n]);
+    }
+    if (lane == 0 && a.n_quartets && nsurv) atomicAdd(a.n_quartets, nsurv);
     if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
 }
 
@@ -1940,44 +2323,67 @@ struct ClassTraits {
 
 // What the launcher (jk_launch.hip) needs to know of one class's kernel.
 #define JK_MAX_DEVICES 64
+#define JK_FAST 2
+#define JK_FOUR 5
+#define JK_KERNELS 8
 struct ClassInfo {
     bool lane;
-    const void *fn[2];          // mixed precision / FP64 only (the same for teams)
-    int threads;
-    size_t lds_static;
+    // two wavefronts per work item: FP32 and FP64 queues, FP64 only (the same for
+    // teams), one density in FP64: J and K, J, K (JK_FAST + 0, 1, 2); four
+    // wavefronts (JK_FOUR on): FP64 only, J and K, K; NULL where the class has none
+    const void *fn[JK_KERNELS];
+    int threads[JK_KERNELS];
+    size_t lds_static[JK_KERNELS];
     int nfij;                   // rows of the K rows
     double cost;                // rough work of one primitive quartet
     // workgroups per CU without dynamic LDS, per device (0: not yet asked);
     // a property of the compiled kernel
-    std::atomic<int> *occ[2];
+    std::atomic<int> *occ[JK_KERNELS];
 };
 
 template <int LI, int LJ, int LK, int LL>
 static const ClassInfo *class_info()
 {
-    static std::atomic<int> occ[2][JK_MAX_DEVICES];
+    static std::atomic<int> occ[JK_KERNELS][JK_MAX_DEVICES];
     using T = ClassTraits<LI, LJ, LK, LL>;
     static const ClassInfo info = [] {
         ClassInfo c;
         c.lane = T::LANE;
         c.nfij = ncart(LI) + ncart(LJ);
         c.cost = T::N * (3. * T::NF + 9. * T::GS) + 200.;
-        c.occ[0] = occ[0];
-        c.occ[1] = occ[1];
+        for (int n = 0; n < JK_KERNELS; ++n) { c.occ[n] = occ[n]; c.fn[n] = nullptr; }
         if constexpr (T::LANE) {
-            c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0>;
-            c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1>;
-            c.threads = LANE_WAVES * WAVE;
-            c.lds_static = sizeof(uint32_t) * LANE_WAVES * 2 * 2 * WAVE +
-                           sizeof(double) * MomentRows<T::N>::SIZE;
+            constexpr bool FAST = LaneFast<LI, LJ, LK, LL>::ON;
+            c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0, 2>;
+            c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 2>;
+            if constexpr (FAST) {
+                c.fn[2] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2>;
+                c.fn[3] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2>;
+                c.fn[4] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2>;
+            }
+            if constexpr (FourWaves<LI, LJ, LK, LL>::ON) {
+                c.fn[5] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 4>;
+                if constexpr (FAST) {
+                    c.fn[6] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4>;
+                    c.fn[7] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4>;
+                }
+            }
+            for (int n = 0; n < JK_KERNELS; ++n) {
+                const int nw = n < JK_FOUR ? 2 : 4;
+                const bool fast = n >= JK_FAST && n != JK_FOUR;
+                c.threads[n] = nw * WAVE;
+                c.lds_static[n] = sizeof(uint32_t) * nw * 2 * 2 * WAVE +
+                                  sizeof(double) * MomentRows<T::N>::SIZE +
+                                  (fast ? 2 * sizeof(double) * ncart(LI) * ncart(LJ) + 32 : 0);
+            }
         } else {
             using S = TeamShape<LI, LJ, LK, LL>;
             c.fn[0] = c.fn[1] = (const void *)jk_team_kernel<LI, LJ, LK, LL>;
-            c.threads = S::TB;
             // queue, wave counts, stop flag, team buffers
-            c.lds_static = sizeof(uint32_t) * 2 * S::TB + sizeof(int) * (S::TB / WAVE + 2) +
-                           sizeof(double) * (S::NQ * (S::PER_QB + S::DSZ) + S::NFI * S::NFJ) +
-                           256;
+            const size_t lds = sizeof(uint32_t) * 2 * S::TB + sizeof(int) * (S::TB / WAVE + 2) +
+                               sizeof(double) * (S::NQ * (S::PER_QB + S::DSZ) +
+                                                 S::NFI * S::NFJ) + 256;
+            for (int n = 0; n < JK_KERNELS; ++n) { c.lds_static[n] = lds; c.threads[n] = S::TB; }
         }
         return c;
     }();

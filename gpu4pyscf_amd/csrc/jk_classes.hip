@@ -1,15 +1,15 @@
 // Instantiates the class kernels of one part of the angular-class list;
-// compiled once per part (-DJK_PART=0..4) so that the parts build in
-// parallel.  Parts: 0 = li <= 2, then li = 3 split by lj = 0, 1, 2, 3.
+// compiled once per part (-DJK_PART=0..7) so that the parts build in
+// parallel.  Parts: 0 = li <= 1, 1 to 3 = li 2 by lj, 4 to 7 = li 3 by lj.
 #include "jk_class_kernels.h"
 
 #ifndef JK_PART
-#error "JK_PART must be defined (0..4)"
+#error "JK_PART must be defined (0..7)"
 #endif
 
 static constexpr bool in_part(int li, int lj)
 {
-    return JK_PART == 0 ? li <= 2 : (li == 3 && lj == JK_PART - 1);
+    return JK_PART == (li <= 1 ? 0 : li == 2 ? 1 + lj : 4 + lj);
 }
 
 template <int I, int J, int K, int L>

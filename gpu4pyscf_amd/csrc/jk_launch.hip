@@ -13,6 +13,9 @@ const ClassInfo *jk_class_info_part1(int key);
 const ClassInfo *jk_class_info_part2(int key);
 const ClassInfo *jk_class_info_part3(int key);
 const ClassInfo *jk_class_info_part4(int key);
+const ClassInfo *jk_class_info_part5(int key);
+const ClassInfo *jk_class_info_part6(int key);
+const ClassInfo *jk_class_info_part7(int key);
 
 #define JK_TEMPLATED_LMAX 3
 // LDS bytes a workgroup may use (static + dynamic): the device limit, capped
@@ -21,6 +24,9 @@ const ClassInfo *jk_class_info_part4(int key);
 #define JK_LDS_CAP (64 * 1024)
 // work items per launch that the kl chunks of the per-lane gradient aim at
 #define IP1_ITEMS 4096
+// kl pairs from which a work item has enough survivors for four wavefronts
+// (16 waters, J only: 50 -> 52 ms with four; 8 waters def2-SVP: 2.07 -> 2.46)
+#define FOUR_MIN_KL 1024
 // LDS of a gfx950 CU is handed out in units of this many bytes
 #define JK_LDS_UNIT 1280
 
@@ -28,7 +34,8 @@ static const ClassInfo *class_info_of(int key)
 {
     const ClassInfo *(*const parts[])(int) = {jk_class_info_part0, jk_class_info_part1,
                                               jk_class_info_part2, jk_class_info_part3,
-                                              jk_class_info_part4};
+                                              jk_class_info_part4, jk_class_info_part5,
+                                              jk_class_info_part6, jk_class_info_part7};
     for (auto f : parts)
         if (const ClassInfo *c = f(key)) return c;
     return nullptr;
@@ -63,16 +70,16 @@ static DeviceLimits device_limits()
 
 // Workgroups per CU of a class kernel with `bytes` of dynamic LDS: by its
 // registers (asked once per kernel and device) and by the LDS of a CU.
-static int blocks_per_cu(const ClassInfo &c, int pm, size_t bytes, const DeviceLimits &lim)
+static int blocks_per_cu(const ClassInfo &c, int f, size_t bytes, const DeviceLimits &lim)
 {
-    int nb = lim.dev >= 0 ? c.occ[pm][lim.dev].load(std::memory_order_relaxed) : 0;
+    int nb = lim.dev >= 0 ? c.occ[f][lim.dev].load(std::memory_order_relaxed) : 0;
     if (nb == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, c.fn[pm], c.threads, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, c.fn[f], c.threads[f], 0) !=
                 hipSuccess || nb < 1)
             nb = 1;
-        if (lim.dev >= 0) c.occ[pm][lim.dev].store(nb, std::memory_order_relaxed);
+        if (lim.dev >= 0) c.occ[f][lim.dev].store(nb, std::memory_order_relaxed);
     }
-    const size_t lds = (c.lds_static + bytes + JK_LDS_UNIT - 1) / JK_LDS_UNIT * JK_LDS_UNIT;
+    const size_t lds = (c.lds_static[f] + bytes + JK_LDS_UNIT - 1) / JK_LDS_UNIT * JK_LDS_UNIT;
     const int by_lds = (int)(lim.lds_cu / lds);
     return std::max(1, std::min(nb, by_lds));
 }
@@ -93,8 +100,8 @@ struct Item {
 // CU can hold with that LDS, then whole groups before windows, then with
 // density rows before without.  kl_win_policy 1 takes the windows whenever
 // their rows fit.
-static void plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int pm,
-                      const DeviceLimits &lim, Item &it)
+static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int f,
+                           const DeviceLimits &lim, Item &it)
 {
     // whole kl lists per work item unless that leaves the GPU idle
     int nchunks = (LANE_ITEMS + k.npairs_ij - 1) / k.npairs_ij;
@@ -105,29 +112,36 @@ static void plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
     it.blocks = (long)k.npairs_ij * nchunks;
     it.d.use_lds = 0;
     it.lds = 0;
+    // the fast kernels' copy of the ij primitives
+    const bool fast = f >= JK_FAST && f != JK_FOUR;
+    const size_t pij = fast ? (size_t)k.iprim * k.jprim * PIJ_LDS * sizeof(double) : 0;
     const JKWindows &w = k.kl_win[0];
     const long blocks_w = w.win ? (long)k.npairs_ij * w.n_win : 0;
     const bool have_win = w.win && blocks_w <= INT_MAX && LANE_KROWS >= 2;
     long best_key = -1;
     for (int win = 0; win < (have_win ? 2 : 1); ++win) {
         const int kn = win ? w.width : k.k_nao, ln = win ? 0 : k.l_nao;
-        for (int dr = (LANE_DROWS ? 1 : 0); dr >= 0; --dr) {
+        for (int dr = (LANE_DROWS || fast ? 1 : 0); dr >= (fast ? 1 : 0); --dr) {
             size_t bytes = 0;
             int mode = 0;
-            if (a.vk && a.n_dm == 1 && kn >= 0 && ln >= 0 && kn + ln > 0) {
+            if (fast && !a.vk) {
+                bytes = pij;
+                if (c.lds_static[f] + bytes > lim.lds_block) continue;
+            } else if (a.vk && a.n_dm == 1 && kn >= 0 && ln >= 0 && kn + ln > 0) {
                 const size_t both = (size_t)c.nfij * (kn + ln) * sizeof(double);
                 const size_t lonly = (size_t)c.nfij * ln * sizeof(double);
-                if (LANE_KROWS >= 2 && dr && 2 * both + c.lds_static <= lim.lds_block) {
-                    mode = 2 | KR_DROWS; bytes = 2 * both;
-                } else if (LANE_KROWS >= 2 && !dr && both + c.lds_static <= lim.lds_block) {
+                if (LANE_KROWS >= 2 && dr && 2 * both + pij + c.lds_static[f] <= lim.lds_block) {
+                    mode = 2 | KR_DROWS; bytes = 2 * both + pij;
+                } else if (LANE_KROWS >= 2 && !dr && both + c.lds_static[f] <= lim.lds_block) {
                     mode = 2; bytes = both;
                 } else if (!win && LANE_KROWS >= 1 && ln > 0 &&
-                           lonly + c.lds_static <= lim.lds_block) {
+                           lonly + c.lds_static[f] <= lim.lds_block) {
                     mode = 1; bytes = lonly;
                 }
             }
             if (win && (mode & KR_MODE_MASK) != 2) continue;
-            const int nb = blocks_per_cu(c, pm, bytes, lim);
+            if (fast && a.vk && !(mode & KR_DROWS)) continue;
+            const int nb = blocks_per_cu(c, f, bytes, lim);
             long key = ((long)(mode & KR_MODE_MASK) << 24) | ((long)nb << 8) |
                        ((win ? 0 : 1) << 1) | (dr ? 1 : 0);
             if (a.kl_win_policy == 1 && win) key |= 1L << 30;
@@ -143,6 +157,24 @@ static void plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
         it.d.pairs_kl = w.pairs; it.d.q_kl = w.q; it.d.pdata_kl = w.pdata; it.d.win = w.win;
         it.blocks = blocks_w;
     }
+    return best_key >= 0;
+}
+
+// A build of one density in FP64 runs on the kernels compiled for it (JK_FAST:
+// all rows and the ij primitives in LDS) when their LDS fits; returns the
+// kernel, an index of ClassInfo.fn.
+static int plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int pm,
+                     const DeviceLimits &lim, Item &it)
+{
+    const int what = a.vk ? (a.vj ? 0 : 2) : 1;
+    const bool fast = pm == 1 && a.n_dm == 1;
+    const bool four = fast && a.vk && k.npairs_kl >= FOUR_MIN_KL;
+    // in order of preference
+    const int tries[] = {four ? JK_FOUR + (a.vj ? 1 : 2) : -1, fast ? JK_FAST + what : -1,
+                         four ? JK_FOUR : -1, pm};
+    for (int f : tries)
+        if (f >= 0 && c.fn[f] && plan_lane_rows(a, k, c, f, lim, it)) return f;
+    return pm;
 }
 
 static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
@@ -158,7 +190,7 @@ static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
         // enough work items to fill the GPU
         const size_t bytes = sizeof(double) * c.nfij * (size_t)w.width;
         const long blocks_w = (long)k.npairs_ij * w.n_win;
-        if (bytes + c.lds_static <= lim.lds_block && blocks_w <= INT_MAX &&
+        if (bytes + c.lds_static[1] <= lim.lds_block && blocks_w <= INT_MAX &&
             (a.kl_win_policy == 1 || blocks_w >= TEAM_KWIN_MIN_ITEMS)) {
             it.d.pairs_kl = w.pairs; it.d.q_kl = w.q; it.d.pdata_kl = w.pdata; it.d.win = w.win;
             it.d.use_lds = 2 | KR_WIN;
@@ -168,7 +200,7 @@ static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
     }
     if (!(it.d.use_lds & KR_WIN) && TEAM_KROWS >= 1 && a.vk && a.n_dm == 1 && k.l_nao > 0) {
         const size_t bytes = sizeof(double) * c.nfij * (size_t)k.l_nao;
-        if (bytes + c.lds_static <= lim.lds_block) { it.d.use_lds = 1; it.lds = bytes; }
+        if (bytes + c.lds_static[1] <= lim.lds_block) { it.d.use_lds = 1; it.lds = bytes; }
     }
     it.per_cu = blocks_per_cu(c, 1, it.lds, lim);
 }
@@ -280,9 +312,11 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
         } else {
             const ClassInfo *c = class_info_of(key);
             if (!c) return hipErrorNotSupported;
-            kern = {c->fn[pm], c->threads};
-            if (c->lane) plan_lane(a, k, *c, pm, lim, it);
+            int f = pm;
+            if (c->lane) f = plan_lane(a, k, *c, pm, lim, it);
             else plan_team(a, k, *c, lim, it);
+            kern = {c->fn[f], c->threads[f]};
+            key = key * 8 + f;
             it.cost = quartets * c->cost;
         }
         if (it.blocks > INT_MAX) return hipErrorInvalidConfiguration;
