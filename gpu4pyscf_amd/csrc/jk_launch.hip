@@ -115,7 +115,12 @@ static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInf
     // the fast kernels' copy of the ij primitives
     const bool fast = f >= JK_FAST && f != JK_FOUR;
     const size_t pij = fast ? (size_t)k.iprim * k.jprim * PIJ_LDS * sizeof(double) : 0;
-    const JKWindows &w = k.kl_win[0];
+    // bra blocks of 9 AOs and more on the narrower windows: rows over the wider
+    // ones leave one workgroup per CU, or do not fit (48 waters def2-TZVP, one
+    // stream, ms, 256 -> 128 AOs: (dp|ps) 34.4 -> 25.6, (fp|ps) 30.9 -> 19.7,
+    // (fs|ds) 23.0 -> 17.0, (fp|ss) 17.4 -> 9.1, (dp|ds) 14.8 -> 10.9; 4 to 7 AOs:
+    // (ps|ps) 55.9 -> 62.4, (ds|ps) 35.1 -> 41.1, (ds|pp) 31.3 -> 36.2)
+    const JKWindows &w = k.kl_win[fast && c.nfij >= 9 && k.kl_win[1].win ? 1 : 0];
     const long blocks_w = w.win ? (long)k.npairs_ij * w.n_win : 0;
     const bool have_win = w.win && blocks_w <= INT_MAX && LANE_KROWS >= 2;
     long best_key = -1;

@@ -29,9 +29,10 @@ from gpu4pyscf_amd.lib import clib
 __all__ = ['get_jk', 'get_j', 'get_k', '_VHFOpt']
 
 TILE = 12                 # pair enumeration tile, gpu4pyscf/scf/jk.py:51
-KL_WINDOW_AO = 256        # widest kl column window (AOs of k, and of l), per-lane kernels
-KL_WINDOW_AO_TEAM = 0     # the same for the team kernels (0: none; they run faster
-                          # with K atomics than with LDS rows over windows)
+# widest kl column windows (AOs of k, and of l) for the LDS K rows of the per-lane
+# kernels: bra blocks below 9 AOs, and larger ones
+KL_WINDOW_AO = 256
+KL_WINDOW_AO_NARROW = 128
 Q_COND_MARGIN = 4.        # bin width of the descending q_cond ordering
 LMAX = clib.JK_LMAX
 
@@ -229,14 +230,15 @@ class _VHFOpt:
         self.task_filter = None
         # kl column windows: group pairs wider than kl_window_ao AOs in k or
         # l are split into windows of at most that many AOs each, so that a
-        # work item (ij pair, window) keeps its K rows in LDS; the per-lane
-        # kernels use kl_window_ao, the team kernels kl_window_ao_team (the
-        # launcher decides per launch; kl_win_policy 1: always when they fit)
+        # work item (ij pair, window) keeps its K rows in LDS; kl_window_ao for
+        # the per-lane kernels, kl_window_ao_team for those with many rows, and
+        # for the team kernels under kl_win_policy 1 (the launcher decides per
+        # launch; policy 1: always when they fit)
         # tasks run with bra and ket exchanged where that puts the larger
         # block on the bra side (JKBuildArgs.swap_ijkl)
         self.swap_tasks = True
         self.kl_window_ao = KL_WINDOW_AO
-        self.kl_window_ao_team = KL_WINDOW_AO_TEAM
+        self.kl_window_ao_team = KL_WINDOW_AO_NARROW
         self.kl_win_policy = 0
 
     def profile_results(self):

@@ -137,9 +137,10 @@ typedef struct {
      * or D_jl, vj must be NULL (RYS_build_k, create_tasks.cu:86-93). */
     int screen;
     /* Column windows of the kl list (JKWindows), for the K rows of a work
-     * item accumulated in LDS: kl_win[0] for the per-lane kernels, kl_win[1]
-     * (narrower) for the team kernels; a NULL win means none.
-     * kl_win_policy 0: the launcher picks, per launch, whole groups or
+     * item accumulated in LDS: kl_win[0], and narrower ones kl_win[1] for the
+     * per-lane kernels of bra blocks of 9 AOs and more and for the team
+     * kernels; a NULL win means none.
+     * kl_win_policy 0: the launcher picks, per task, whole groups or
      * windows: first the choice that keeps all four K blocks in LDS, then
      * the one whose LDS leaves the most workgroups per CU (the team kernels
      * take kl_win[1] only under policy 1); 1: windows whenever their rows
