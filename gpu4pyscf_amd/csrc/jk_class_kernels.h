@@ -829,7 +829,8 @@ struct TaskDesc {
     int kl_chunk;                   // candidates per work item (not KR_WIN)
     int use_lds;                    // KR_* bits
     int counter;                    // element of the per-task counters
-    uint32_t ls_swap;               // li, lj, lk, ll, 4 bits each, and swap_ijkl << 16
+    // li, lj, lk, ll, 4 bits each, swap_ijkl << 16, first density << 17
+    uint32_t ls_swap;
 };
 struct TaskBatch {
     int n, pad;
@@ -852,7 +853,7 @@ __device__ __forceinline__ T *as_global(T *p)
 // The task of this workgroup: its fields into the launch's arguments;
 // returns the workgroup's index within the task.
 __device__ __forceinline__ int select_task(JKBuildArgs &a, const TaskBatch &b, int &kl_chunk,
-                                           int &use_lds)
+                                           int &use_lds, int &dm0)
 {
     const int blk = blockIdx.x;
     int t = 0;
@@ -861,7 +862,8 @@ __device__ __forceinline__ int select_task(JKBuildArgs &a, const TaskBatch &b, i
     const TaskDesc &d = b.t[t];
     a.li = d.ls_swap & 15; a.lj = d.ls_swap >> 4 & 15;
     a.lk = d.ls_swap >> 8 & 15; a.ll = d.ls_swap >> 12 & 15;
-    a.swap_ijkl = d.ls_swap >> 16;
+    a.swap_ijkl = d.ls_swap >> 16 & 1;
+    dm0 = d.ls_swap >> 17;
     a.pairs_ij = as_global(d.pairs_ij); a.pairs_kl = as_global(d.pairs_kl);
     a.q_ij = as_global(d.q_ij); a.q_kl = as_global(d.q_kl);
     a.pdata_ij = as_global(d.pdata_ij); a.pdata_kl = as_global(d.pdata_kl);
@@ -870,12 +872,20 @@ __device__ __forceinline__ int select_task(JKBuildArgs &a, const TaskBatch &b, i
     a.iprim = d.prims_ij & 0xffff; a.jprim = d.prims_ij >> 16;
     a.kprim = d.prims_kl & 0xffff; a.lprim = d.prims_kl >> 16;
     a.k_ao0 = d.k_ao0; a.k_nao = d.k_nao; a.l_ao0 = d.l_ao0; a.l_nao = d.l_nao;
-    if (a.n_quartets) a.n_quartets += d.counter;
-    if (a.n_quartets_fp32) a.n_quartets_fp32 += d.counter;
-    if (a.quartet_hash) a.quartet_hash += d.counter;
+    // (the launches of the first density count)
+    a.n_quartets = a.n_quartets && dm0 == 0 ? a.n_quartets + d.counter : nullptr;
+    a.n_quartets_fp32 = a.n_quartets_fp32 && dm0 == 0 ? a.n_quartets_fp32 + d.counter : nullptr;
+    a.quartet_hash = a.quartet_hash && dm0 == 0 ? a.quartet_hash + d.counter : nullptr;
     kl_chunk = d.kl_chunk;
     use_lds = d.use_lds;
     return blk - b.block0[t];
+}
+
+__device__ __forceinline__ int select_task(JKBuildArgs &a, const TaskBatch &b, int &kl_chunk,
+                                           int &use_lds)
+{
+    int dm0;
+    return select_task(a, b, kl_chunk, use_lds, dm0);
 }
 
 __device__ __forceinline__ WorkItem work_item(int idx, int npairs_kl, int kl_chunk)
@@ -952,9 +962,17 @@ __device__ __forceinline__ KRows make_krows(double *buf, int use_lds, int nrows,
     return kr;
 }
 
+// the same rows `off` doubles on (another density's)
+__device__ __forceinline__ KRows krows_of(KRows kr, int off)
+{
+    kr.p += off;
+    kr.d += off;
+    return kr;
+}
+
 // copy the density rows (after krows_zero; a barrier must follow)
 __device__ __forceinline__ void krows_load_d(const KRows &kr, int nfi, int nfj, int i0, int j0,
-                                             const JKBuildArgs &a, int tid, int nthreads)
+                                             int nao, const double *dm, int tid, int nthreads)
 {
     if (!kr.dstaged) return;
     lds_double *d = kr.p + (nfi + nfj) * kr.width;
@@ -963,7 +981,7 @@ __device__ __forceinline__ void krows_load_d(const KRows &kr, int nfi, int nfj, 
         int r = n / kr.width, c = n - r * kr.width;
         int row = r < nfi ? i0 + r : j0 + r - nfi;
         int col = c < kr.loff ? kr.k_ao0 + c : kr.l_ao0 + c - kr.loff;
-        d[n] = a.dm[(size_t)row * a.nao + col];
+        d[n] = dm[(size_t)row * nao + col];
     }
 }
 
@@ -976,7 +994,7 @@ __device__ __forceinline__ void krows_zero(const KRows &kr, int nrows, int tid, 
 
 // flush (after a barrier that ends the block's accumulation)
 __device__ __forceinline__ void krows_flush(const KRows &kr, int nfi, int nfj, int i0, int j0,
-                                            const JKBuildArgs &a, int tid, int nthreads)
+                                            int nao, double *vk, int tid, int nthreads)
 {
     if (!kr.on) return;
     const int n_all = (nfi + nfj) * kr.width;
@@ -986,7 +1004,7 @@ __device__ __forceinline__ void krows_flush(const KRows &kr, int nfi, int nfj, i
             int r = n / kr.width, c = n - r * kr.width;
             int row = r < nfi ? i0 + r : j0 + r - nfi;
             int col = c < kr.loff ? kr.k_ao0 + c : kr.l_ao0 + c - kr.loff;
-            atomic_add(a.vk + (size_t)row * a.nao + col, v);
+            atomic_add(vk + (size_t)row * nao + col, v);
         }
     }
 }
@@ -1534,7 +1552,7 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     const KRows kr = make_krows(kacc_dyn, use_lds, NFI + NFJ, wi);
     if (kr.on) {
         krows_zero(kr, NFI + NFJ, threadIdx.x, NW * WAVE);
-        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, NW * WAVE);
+        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, nao, a.dm, threadIdx.x, NW * WAVE);
     }
     load_moment_rows<N>(moment_buf, a.rys, threadIdx.x, NW * WAVE);
     __syncthreads();
@@ -1601,7 +1619,7 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     }
     if (kr.on) {
         __syncthreads();
-        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, threadIdx.x, NW * WAVE);
+        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, nao, a.vk, threadIdx.x, NW * WAVE);
     }
     if (lane == 0) {
         if (a.n_quartets && nsurv) atomicAdd(a.n_quartets, nsurv);
@@ -1610,8 +1628,8 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
     if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
 }
 
-// ---------------------------------------------------------------- one density
-// Per-lane kernel of the FP64 builds of one density with J and K (WJ, WK), J
+// ---------------------------------------------------------------- one or two densities
+// Per-lane kernel of the FP64 builds of ND = 1 or 2 densities with J and K (WJ, WK), J
 // only or K only: what jk_lane_kernel decides at run time -- which matrices,
 // where K is accumulated, the number of densities -- is fixed here, with the K
 // rows and the density rows of the work item in LDS (KR_DROWS), J_ij and D_ij
@@ -1624,6 +1642,9 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
 // 48 waters (def2-TZVP), one stream, ms: (ps|ss) 65.8 -> 58.5,
 // (dp|ps) 40.6 -> 34.3, (dp|ss) 17.0 -> 13.7, (ds|ss) 29.0 -> 24.5, (ds|ps) 38.9 -> 35.4;
 // the whole build on four streams 1000 -> 952.
+// ND densities share the integrals, each with its own rows in LDS; the kernels for
+// any number keep their K rows in HBM (two densities of 8 waters 53.6 -> 36.1 ms,
+// of 12 waters 143 -> 75).
 // Chunked classes with an f shell stay on jk_lane_kernel: the J_kl block held
 // over the chunks costs them more registers than the waits ((fp|fs) 20.8 -> 22.5,
 // (fp|pp) 33.7 -> 34.5, (fp|ds) 29.4 -> 29.9).
@@ -1633,12 +1654,13 @@ struct LaneFast {
 };
 
 struct ItemLds {
-    const lds_double *pij, *dij;
+    const lds_double *pij, *dij;    // D_ij and J_ij: ij_step doubles from density to density
     lds_double *jij;
     const lds_double *rows;
+    int kr_step;                    // K and density rows, from density to density
 };
 
-template <int LI, int LJ, int LK, int LL, bool WJ, bool WK>
+template <int LI, int LJ, int LK, int LL, bool WJ, bool WK, int ND>
 __device__ __forceinline__ void lane_batch_fast(const JKBuildArgs &a, const ShellPair &sp,
                                                 int pkl, uint32_t sh, bool active, int lane,
                                                 const KRows &kr, const ItemLds &it,
@@ -1661,9 +1683,10 @@ __device__ __forceinline__ void lane_batch_fast(const JKBuildArgs &a, const Shel
     // columns of this quartet's k and l AOs in the LDS rows
     const int dk = k0 - kr.k_ao0, dl = kr.loff + l0 - kr.l_ao0;
     const uint32_t off_kl = (uint32_t)k0 * (uint32_t)nao + (uint32_t)l0;
-    double vkl[NFK * NFL];
+    constexpr int NFKL = NFK * NFL;
+    double vkl[ND * NFKL];
 #pragma unroll
-    for (int n = 0; n < NFK * NFL; ++n) vkl[n] = 0.;
+    for (int n = 0; n < ND * NFKL; ++n) vkl[n] = 0.;
     lane_chunks<(NFI + CH - 1) / CH>([&](auto cc) {
         constexpr int I0 = decltype(cc)::value * CH;
         constexpr int I1 = I0 + CH < NFI ? I0 + CH : NFI;
@@ -1675,116 +1698,125 @@ __device__ __forceinline__ void lane_batch_fast(const JKBuildArgs &a, const Shel
                 if constexpr (WJ && I0 == 0) {
                     // J_kl of the previous batch
                     if (pend_off != ~0u) {
-                        double *J = a.vj + pend_off;
 #pragma unroll
-                        for (int n = 0; n < NFK * NFL; ++n)
-                            atomic_add(J + (uint32_t)((n / NFL) * nao + n % NFL), pend[n]);
+                        for (int id = 0; id < ND; ++id) {
+                            double *J = a.vj + (size_t)id * nao * nao + pend_off;
+#pragma unroll
+                            for (int n = 0; n < NFKL; ++n)
+                                atomic_add(J + (uint32_t)((n / NFL) * nao + n % NFL),
+                                           pend[id * NFKL + n]);
+                        }
                     }
                 }
             });
-        if constexpr (WK) {
-            // K_ik += (ij|kl) D_jl ; K_il += (ij|kl) D_jk
 #pragma unroll
-            for (int i = I0; i < I1; ++i) {
-                double kil[NFL], kik[NFK];
+        for (int id = 0; id < ND; ++id) {
+            lds_double *kp = kr.p + id * it.kr_step;
+            const lds_double *kd = kr.d + id * it.kr_step;
+            if constexpr (WK) {
+                // K_ik += (ij|kl) D_jl ; K_il += (ij|kl) D_jk
 #pragma unroll
-                for (int l = 0; l < NFL; ++l) kil[l] = 0.;
+                for (int i = I0; i < I1; ++i) {
+                    double kil[NFL], kik[NFK];
 #pragma unroll
-                for (int k = 0; k < NFK; ++k) kik[k] = 0.;
-                if (active) {
+                    for (int l = 0; l < NFL; ++l) kil[l] = 0.;
 #pragma unroll
-                    for (int j = 0; j < NFJ; ++j) {
-                        const lds_double *dj = kr.d + (NFI + j) * kr.width;
+                    for (int k = 0; k < NFK; ++k) kik[k] = 0.;
+                    if (active) {
 #pragma unroll
-                        for (int k = 0; k < NFK; ++k)
+                        for (int j = 0; j < NFJ; ++j) {
+                            const lds_double *dj = kd + (NFI + j) * kr.width;
 #pragma unroll
-                        for (int l = 0; l < NFL; ++l) {
-                            const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
-                            kil[l] = fma(g, dj[dk + k], kil[l]);
-                            kik[k] = fma(g, dj[dl + l], kik[k]);
+                            for (int k = 0; k < NFK; ++k)
+#pragma unroll
+                            for (int l = 0; l < NFL; ++l) {
+                                const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
+                                kil[l] = fma(g, dj[dk + k], kil[l]);
+                                kik[k] = fma(g, dj[dl + l], kik[k]);
+                            }
                         }
+#pragma unroll
+                        for (int k = 0; k < NFK; ++k) lds_add(kp + i * kr.width + dk + k, kik[k]);
+#pragma unroll
+                        for (int l = 0; l < NFL; ++l) lds_add(kp + i * kr.width + dl + l, kil[l]);
                     }
-#pragma unroll
-                    for (int k = 0; k < NFK; ++k) lds_add(kr.p + i * kr.width + dk + k, kik[k]);
-#pragma unroll
-                    for (int l = 0; l < NFL; ++l) lds_add(kr.p + i * kr.width + dl + l, kil[l]);
                 }
-            }
-            // K_jk += (ij|kl) D_il ; K_jl += (ij|kl) D_ik
+                // K_jk += (ij|kl) D_il ; K_jl += (ij|kl) D_ik
 #pragma unroll
-            for (int j = 0; j < NFJ; ++j) {
-                double kjl[NFL], kjk[NFK];
+                for (int j = 0; j < NFJ; ++j) {
+                    double kjl[NFL], kjk[NFK];
 #pragma unroll
-                for (int l = 0; l < NFL; ++l) kjl[l] = 0.;
+                    for (int l = 0; l < NFL; ++l) kjl[l] = 0.;
 #pragma unroll
-                for (int k = 0; k < NFK; ++k) kjk[k] = 0.;
-                if (active) {
+                    for (int k = 0; k < NFK; ++k) kjk[k] = 0.;
+                    if (active) {
 #pragma unroll
-                    for (int i = I0; i < I1; ++i) {
-                        const lds_double *di = kr.d + i * kr.width;
+                        for (int i = I0; i < I1; ++i) {
+                            const lds_double *di = kd + i * kr.width;
 #pragma unroll
-                        for (int k = 0; k < NFK; ++k)
+                            for (int k = 0; k < NFK; ++k)
 #pragma unroll
-                        for (int l = 0; l < NFL; ++l) {
-                            const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
-                            kjl[l] = fma(g, di[dk + k], kjl[l]);
-                            kjk[k] = fma(g, di[dl + l], kjk[k]);
+                            for (int l = 0; l < NFL; ++l) {
+                                const double g = gout[(((i - I0)*NFJ + j)*NFK + k)*NFL + l];
+                                kjl[l] = fma(g, di[dk + k], kjl[l]);
+                                kjk[k] = fma(g, di[dl + l], kjk[k]);
+                            }
                         }
+                        lds_double *kj = kp + (NFI + j) * kr.width;
+#pragma unroll
+                        for (int k = 0; k < NFK; ++k) lds_add(kj + dk + k, kjk[k]);
+#pragma unroll
+                        for (int l = 0; l < NFL; ++l) lds_add(kj + dl + l, kjl[l]);
                     }
-                    lds_double *kj = kr.p + (NFI + j) * kr.width;
-#pragma unroll
-                    for (int k = 0; k < NFK; ++k) lds_add(kj + dk + k, kjk[k]);
-#pragma unroll
-                    for (int l = 0; l < NFL; ++l) lds_add(kj + dl + l, kjl[l]);
                 }
             }
-        }
-        if constexpr (WJ) {
-            double dkl[NFK * NFL];
-            const double *D = a.dm + off_kl;
+            if constexpr (WJ) {
+                double dkl[NFKL];
+                const double *D = a.dm + (size_t)id * nao * nao + off_kl;
 #pragma unroll
-            for (int n = 0; n < NFK * NFL; ++n) dkl[n] = D[(uint32_t)((n / NFL) * nao + n % NFL)];
-            double vij[NI * NFJ];
+                for (int n = 0; n < NFKL; ++n) dkl[n] = D[(uint32_t)((n / NFL) * nao + n % NFL)];
+                double vij[NI * NFJ];
 #pragma unroll
-            for (int i = I0; i < I1; ++i)
+                for (int i = I0; i < I1; ++i)
 #pragma unroll
-            for (int j = 0; j < NFJ; ++j) {
-                const double d = it.dij[i * NFJ + j];
-                double s = 0.;
+                for (int j = 0; j < NFJ; ++j) {
+                    const double d = it.dij[2 * id * NFI * NFJ + i * NFJ + j];
+                    double s = 0.;
 #pragma unroll
-                for (int n = 0; n < NFK * NFL; ++n) {
-                    const double g = gout[((i - I0)*NFJ + j)*NFK*NFL + n];
-                    s = fma(g, dkl[n], s);
-                    vkl[n] = fma(g, d, vkl[n]);
+                    for (int n = 0; n < NFKL; ++n) {
+                        const double g = gout[((i - I0)*NFJ + j)*NFKL + n];
+                        s = fma(g, dkl[n], s);
+                        vkl[id * NFKL + n] = fma(g, d, vkl[id * NFKL + n]);
+                    }
+                    // (an inactive lane's integrals are zero)
+                    vij[(i - I0)*NFJ + j] = s;
                 }
-                // (an inactive lane's integrals are zero)
-                vij[(i - I0)*NFJ + j] = s;
+                wave_reduce_scatter<NI * NFJ>(vij, lane, [&](int n, double x) {
+                    lds_add(it.jij + 2 * id * NFI * NFJ + I0 * NFJ + n, x);
+                });
             }
-            wave_reduce_scatter<NI * NFJ>(vij, lane, [&](int n, double x) {
-                lds_add(it.jij + I0 * NFJ + n, x);
-            });
         }
     });
     if constexpr (WJ) {
 #pragma unroll
-        for (int n = 0; n < NFK * NFL; ++n) pend[n] = vkl[n];
+        for (int n = 0; n < ND * NFKL; ++n) pend[n] = vkl[n];
         pend_off = active ? off_kl : ~0u;
     }
 }
 
-template <int LI, int LJ, int LK, int LL, bool WJ, bool WK, int NW>
+template <int LI, int LJ, int LK, int LL, bool WJ, bool WK, int NW, int ND>
 __global__ __launch_bounds__((NW * WAVE), (ClassOcc<LI, LJ, LK, LL>::W))
 void jk_lane_fast_kernel(JKBuildArgs a, TaskBatch batch)
 {
-    int kl_chunk, use_lds;
-    const int item = select_task(a, batch, kl_chunk, use_lds);
+    int kl_chunk, use_lds, dm0;
+    const int item = select_task(a, batch, kl_chunk, use_lds, dm0);
     constexpr int NFI = ncart(LI), NFJ = ncart(LJ), NFKL = ncart(LK) * ncart(LL);
     constexpr int N = (LI + LJ + LK + LL) / 2 + 1;
     constexpr int NT = NW * WAVE;
     __shared__ uint32_t queue_all[NW][2][2 * WAVE];
     __shared__ int left[NW];
     __shared__ __align__(16) double moment_buf[MomentRows<N>::SIZE];
-    __shared__ double ij_buf[2][NFI * NFJ];
+    __shared__ double ij_buf[2 * ND][NFI * NFJ];
     extern __shared__ __align__(16) double fast_dyn[];
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
@@ -1792,6 +1824,10 @@ void jk_lane_fast_kernel(JKBuildArgs a, TaskBatch batch)
     uint32_t *queue = queue_all[wid][0], *queue_sh = queue_all[wid][1];
     const int nbas = a.nbas, nao = a.nao;
     select_replica(a);
+    const size_t nao2 = (size_t)nao * nao;
+    a.dm += dm0 * nao2;
+    if constexpr (WJ) a.vj += dm0 * nao2;
+    if constexpr (WK) a.vk += dm0 * nao2;
     const WorkItem wi = work_item(a, item, kl_chunk, use_lds);
     const uint32_t bas_ij = a.pairs_ij[wi.pij];
     const float q_ij = a.q_ij[wi.pij];
@@ -1809,24 +1845,32 @@ void jk_lane_fast_kernel(JKBuildArgs a, TaskBatch batch)
     it.jij = (lds_double *)ij_buf[1];
     it.rows = (lds_double *)moment_buf;
     const KRows kr = make_krows(fast_dyn + nij * PIJ_LDS, WK ? 2 | KR_DROWS : 0, NFI + NFJ, wi);
+    it.kr_step = 2 * (NFI + NFJ) * kr.width;
     if constexpr (WK) {
-        krows_zero(kr, NFI + NFJ, tid, NT);
-        krows_load_d(kr, NFI, NFJ, sp.i0, sp.j0, a, tid, NT);
+#pragma unroll
+        for (int id = 0; id < ND; ++id) {
+            const KRows krd = krows_of(kr, id * it.kr_step);
+            krows_zero(krd, NFI + NFJ, tid, NT);
+            krows_load_d(krd, NFI, NFJ, sp.i0, sp.j0, nao, a.dm + id * nao2, tid, NT);
+        }
     }
     stage_pij(pij, a.pdata_ij + (size_t)wi.pij * nij * PREC, nij, sp.ri, tid, NT);
     load_moment_rows<N>(moment_buf, a.rys, tid, NT);
     for (int n = tid; n < NFI * NFJ; n += NT) {
-        ij_buf[0][n] = a.dm[(size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ];
-        ij_buf[1][n] = 0.;
+#pragma unroll
+        for (int id = 0; id < ND; ++id) {
+            ij_buf[2 * id][n] = a.dm[id * nao2 + (size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ];
+            ij_buf[2 * id + 1][n] = 0.;
+        }
     }
     __syncthreads();
     int qn = 0;
     unsigned long long nsurv = 0, hsum = 0;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    double pend[WJ ? NFKL : 1];
+    double pend[WJ ? ND * NFKL : 1];
     uint32_t pend_off = ~0u;
 #pragma unroll
-    for (int n = 0; n < (WJ ? NFKL : 1); ++n) pend[n] = 0.;
+    for (int n = 0; n < (WJ ? ND * NFKL : 1); ++n) pend[n] = 0.;
     // floor(b / nbas) of a pair id: the reciprocal's estimate is at most one
     // too large
     const uint32_t nbas_inv = 0xffffffffu / (uint32_t)nbas + 1u;
@@ -1882,24 +1926,32 @@ void jk_lane_fast_kernel(JKBuildArgs a, TaskBatch batch)
             for (w = 0; n >= left[w]; ++w) n -= left[w];
             last = true;
         }
-        lane_batch_fast<LI, LJ, LK, LL, WJ, WK>(a, sp, queue_all[w][0][n], queue_all[w][1][n],
-                                                active, lane, kr, it, pend, pend_off);
+        lane_batch_fast<LI, LJ, LK, LL, WJ, WK, ND>(a, sp, queue_all[w][0][n], queue_all[w][1][n],
+                                                    active, lane, kr, it, pend, pend_off);
         wave_sync();
     }
     if constexpr (WJ) {
         if (pend_off != ~0u) {
             constexpr int NFL = ncart(LL);
-            double *J = a.vj + pend_off;
 #pragma unroll
-            for (int n = 0; n < NFKL; ++n)
-                atomic_add(J + (uint32_t)((n / NFL) * nao + n % NFL), pend[n]);
+            for (int n = 0; n < ND * NFKL; ++n)
+                atomic_add(a.vj + (n / NFKL) * nao2 + pend_off +
+                               (uint32_t)((n % NFKL / NFL) * nao + n % NFL), pend[n]);
         }
     }
     __syncthreads();
-    if constexpr (WK) krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, tid, NT);
+    if constexpr (WK) {
+#pragma unroll
+        for (int id = 0; id < ND; ++id)
+            krows_flush(krows_of(kr, id * it.kr_step), NFI, NFJ, sp.i0, sp.j0, nao,
+                        a.vk + id * nao2, tid, NT);
+    }
     if constexpr (WJ) {
-        for (int n = tid; n < NFI * NFJ; n += NT)
-            atomic_add(a.vj + (size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ, ij_buf[1][n]);
+#pragma unroll
+        for (int id = 0; id < ND; ++id)
+            for (int n = tid; n < NFI * NFJ; n += NT)
+                atomic_add(a.vj + id * nao2 + (size_t)(sp.i0 + n / NFJ) * nao + sp.j0 + n % NFJ,
+                           ij_buf[2 * id + 1][n]);
     }
     if (lane == 0 && a.n_quartets && nsurv) atomicAdd(a.n_quartets, nsurv);
     if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
@@ -2300,7 +2352,7 @@ void jk_team_kernel(JKBuildArgs a, TaskBatch batch)
         atomic_add(a.vj + (sp.i0 + irow)*nao + sp.j0 + jrow, vj_row);
     if (kr.on) {
         __syncthreads();
-        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, a, tid, TB);
+        krows_flush(kr, NFI, NFJ, sp.i0, sp.j0, nao, a.vk, tid, TB);
     }
     if (a.n_quartets && tid == 0 && nsurv) atomicAdd(a.n_quartets, nsurv);
     if (a.quartet_hash && hsum) atomicAdd(a.quartet_hash, hsum);
@@ -2325,12 +2377,25 @@ struct ClassTraits {
 #define JK_MAX_DEVICES 64
 #define JK_FAST 2
 #define JK_FOUR 5
-#define JK_KERNELS 8
+#define JK_TWO 8
+#define JK_KERNELS 13
+// wavefronts of kernel n of the per-lane classes, and densities of a fast one
+// (0: any number)
+static constexpr int lane_waves(int n)
+{
+    return (n >= JK_FOUR && n < JK_TWO) || n >= JK_TWO + 3 ? 4 : 2;
+}
+static constexpr int lane_densities(int n)
+{
+    return n >= JK_TWO ? 2 : n >= JK_FAST && n != JK_FOUR ? 1 : 0;
+}
 struct ClassInfo {
     bool lane;
     // two wavefronts per work item: FP32 and FP64 queues, FP64 only (the same for
     // teams), one density in FP64: J and K, J, K (JK_FAST + 0, 1, 2); four
-    // wavefronts (JK_FOUR on): FP64 only, J and K, K; NULL where the class has none
+    // wavefronts (JK_FOUR on): FP64 only, J and K, K; two densities in FP64 (JK_TWO
+    // on): as JK_FAST, and J and K, K with four wavefronts; NULL where the class has
+    // none
     const void *fn[JK_KERNELS];
     int threads[JK_KERNELS];
     size_t lds_static[JK_KERNELS];
@@ -2357,24 +2422,29 @@ static const ClassInfo *class_info()
             c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0, 2>;
             c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 2>;
             if constexpr (FAST) {
-                c.fn[2] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2>;
-                c.fn[3] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2>;
-                c.fn[4] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2>;
+                c.fn[2] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2, 1>;
+                c.fn[3] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2, 1>;
+                c.fn[4] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 1>;
+                c.fn[8] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2, 2>;
+                c.fn[9] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2, 2>;
+                c.fn[10] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 2>;
             }
             if constexpr (FourWaves<LI, LJ, LK, LL>::ON) {
                 c.fn[5] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 4>;
                 if constexpr (FAST) {
-                    c.fn[6] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4>;
-                    c.fn[7] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4>;
+                    c.fn[6] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4, 1>;
+                    c.fn[7] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 1>;
+                    c.fn[11] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4, 2>;
+                    c.fn[12] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 2>;
                 }
             }
             for (int n = 0; n < JK_KERNELS; ++n) {
-                const int nw = n < JK_FOUR ? 2 : 4;
-                const bool fast = n >= JK_FAST && n != JK_FOUR;
+                const int nw = lane_waves(n), nd = lane_densities(n);
                 c.threads[n] = nw * WAVE;
                 c.lds_static[n] = sizeof(uint32_t) * nw * 2 * 2 * WAVE +
                                   sizeof(double) * MomentRows<T::N>::SIZE +
-                                  (fast ? 2 * sizeof(double) * ncart(LI) * ncart(LJ) + 32 : 0);
+                                  2 * nd * sizeof(double) * ncart(LI) * ncart(LJ) +
+                                  (nd ? 32 : 0);
             }
         } else {
             using S = TeamShape<LI, LJ, LK, LL>;

@@ -27,6 +27,8 @@ const ClassInfo *jk_class_info_part7(int key);
 // kl pairs from which a work item has enough survivors for four wavefronts
 // (16 waters, J only: 50 -> 52 ms with four; 8 waters def2-SVP: 2.07 -> 2.46)
 #define FOUR_MIN_KL 1024
+// densities that the descriptor of a work item can name (TaskDesc.ls_swap)
+#define FAST_DM_MAX 32767
 // LDS of a gfx950 CU is handed out in units of this many bytes
 #define JK_LDS_UNIT 1280
 
@@ -113,14 +115,15 @@ static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInf
     it.d.use_lds = 0;
     it.lds = 0;
     // the fast kernels' copy of the ij primitives
-    const bool fast = f >= JK_FAST && f != JK_FOUR;
+    const int nd = lane_densities(f);
+    const bool fast = nd > 0;
     const size_t pij = fast ? (size_t)k.iprim * k.jprim * PIJ_LDS * sizeof(double) : 0;
     // bra blocks of 9 AOs and more on the narrower windows: rows over the wider
     // ones leave one workgroup per CU, or do not fit (48 waters def2-TZVP, one
     // stream, ms, 256 -> 128 AOs: (dp|ps) 34.4 -> 25.6, (fp|ps) 30.9 -> 19.7,
     // (fs|ds) 23.0 -> 17.0, (fp|ss) 17.4 -> 9.1, (dp|ds) 14.8 -> 10.9; 4 to 7 AOs:
     // (ps|ps) 55.9 -> 62.4, (ds|ps) 35.1 -> 41.1, (ds|pp) 31.3 -> 36.2)
-    const JKWindows &w = k.kl_win[fast && c.nfij >= 9 && k.kl_win[1].win ? 1 : 0];
+    const JKWindows &w = k.kl_win[fast && c.nfij * nd >= 9 && k.kl_win[1].win ? 1 : 0];
     const long blocks_w = w.win ? (long)k.npairs_ij * w.n_win : 0;
     const bool have_win = w.win && blocks_w <= INT_MAX && LANE_KROWS >= 2;
     long best_key = -1;
@@ -132,8 +135,8 @@ static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInf
             if (fast && !a.vk) {
                 bytes = pij;
                 if (c.lds_static[f] + bytes > lim.lds_block) continue;
-            } else if (a.vk && a.n_dm == 1 && kn >= 0 && ln >= 0 && kn + ln > 0) {
-                const size_t both = (size_t)c.nfij * (kn + ln) * sizeof(double);
+            } else if (a.vk && (fast || a.n_dm == 1) && kn >= 0 && ln >= 0 && kn + ln > 0) {
+                const size_t both = (size_t)c.nfij * (kn + ln) * sizeof(double) * (fast ? nd : 1);
                 const size_t lonly = (size_t)c.nfij * ln * sizeof(double);
                 if (LANE_KROWS >= 2 && dr && 2 * both + pij + c.lds_static[f] <= lim.lds_block) {
                     mode = 2 | KR_DROWS; bytes = 2 * both + pij;
@@ -165,18 +168,30 @@ static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInf
     return best_key >= 0;
 }
 
-// A build of one density in FP64 runs on the kernels compiled for it (JK_FAST:
-// all rows and the ij primitives in LDS) when their LDS fits; returns the
-// kernel, an index of ClassInfo.fn.
-static int plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int pm,
+// A build in FP64 runs on the kernels compiled for one or two densities
+// (JK_FAST, JK_TWO: all rows and the ij primitives in LDS) when their LDS fits;
+// returns the kernel, an index of ClassInfo.fn.  n_dm: densities still to do.
+static int plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, int pm, int n_dm,
                      const DeviceLimits &lim, Item &it)
 {
     const int what = a.vk ? (a.vj ? 0 : 2) : 1;
-    const bool fast = pm == 1 && a.n_dm == 1;
+    // Several densities: only where the last one of an odd number fits too, and
+    // not in several launches of a task that leaves CUs idle, which take the
+    // time of one each (1 water def2-TZVP, three densities: 7.6 -> 10.6 ms).
+    // Two densities, ms, any-number kernel -> this: 8 waters def2-SVP 6.6 -> 3.4,
+    // 8 and 12 waters def2-TZVP 53.6 -> 36.1 and 143 -> 75; 12 waters in two
+    // launches of one density 92.
+    Item one = it;
+    const bool fast = pm == 1 && (a.n_dm == 1 ||
+                                  (a.n_dm <= FAST_DM_MAX && c.fn[JK_FAST + what] &&
+                                   plan_lane_rows(a, k, c, JK_FAST + what, lim, one) &&
+                                   (a.n_dm == 2 || one.blocks > lim.cus)));
+    const bool two = fast && n_dm >= 2;
     const bool four = fast && a.vk && k.npairs_kl >= FOUR_MIN_KL;
     // in order of preference
-    const int tries[] = {four ? JK_FOUR + (a.vj ? 1 : 2) : -1, fast ? JK_FAST + what : -1,
-                         four ? JK_FOUR : -1, pm};
+    const int tries[] = {two && four ? JK_TWO + (a.vj ? 3 : 4) : -1, two ? JK_TWO + what : -1,
+                         four ? JK_FOUR + (a.vj ? 1 : 2) : -1, fast ? JK_FAST + what : -1,
+                         four && a.n_dm == 1 ? JK_FOUR : -1, pm};
     for (int f : tries)
         if (f >= 0 && c.fn[f] && plan_lane_rows(a, k, c, f, lim, it)) return f;
     return pm;
@@ -276,6 +291,16 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
     struct Group { Kernel k; std::vector<Item> items; };
     std::map<int, Group> by_kernel;
     std::vector<int> order;
+    auto add = [&](int key, const Kernel &kern, const Item &it) {
+        if (it.blocks > INT_MAX) return false;
+        Group &g = by_kernel[key];
+        if (g.items.empty()) {
+            order.push_back(key);
+            g.k = kern;
+        }
+        g.items.push_back(it);
+        return true;
+    };
     for (int t = ntasks - 1; t >= 0; --t) {
         const JKTask &k = tasks[t];
         if (k.npairs_ij <= 0 || k.npairs_kl <= 0) continue;
@@ -317,20 +342,25 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
         } else {
             const ClassInfo *c = class_info_of(key);
             if (!c) return hipErrorNotSupported;
-            int f = pm;
-            if (c->lane) f = plan_lane(a, k, *c, pm, lim, it);
-            else plan_team(a, k, *c, lim, it);
-            kern = {c->fn[f], c->threads[f]};
-            key = key * 8 + f;
             it.cost = quartets * c->cost;
+            if (c->lane) {
+                // the fast kernels in as many launches as the densities take
+                for (int dm0 = 0; dm0 < a.n_dm;) {
+                    Item part = it;
+                    const int f = plan_lane(a, k, *c, pm, a.n_dm - dm0, lim, part);
+                    const int nd = lane_densities(f);
+                    if (nd) part.d.ls_swap |= (uint32_t)dm0 << 17;
+                    if (!add(key * JK_KERNELS + f, {c->fn[f], c->threads[f]}, part))
+                        return hipErrorInvalidConfiguration;
+                    dm0 += nd ? nd : a.n_dm;
+                }
+                continue;
+            }
+            plan_team(a, k, *c, lim, it);
+            kern = {c->fn[pm], c->threads[pm]};
+            key = key * JK_KERNELS + pm;
         }
-        if (it.blocks > INT_MAX) return hipErrorInvalidConfiguration;
-        Group &g = by_kernel[key];
-        if (g.items.empty()) {
-            order.push_back(key);
-            g.k = kern;
-        }
-        g.items.push_back(it);
+        if (!add(key, kern, it)) return hipErrorInvalidConfiguration;
     }
     std::vector<Launch> launches;
     for (int key : order)
