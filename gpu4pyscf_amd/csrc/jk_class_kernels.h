@@ -1087,18 +1087,34 @@ __device__ __forceinline__ void stage_pij(lds_double *dst, const double *rec, in
     }
 }
 
+// Operator of a launch (JKBuildArgs.omega, full): erf(omega r)/r for omega2 > 0,
+// else 1/r; with full != 0 also full / r, as a second set of roots of every
+// primitive quartet.  The two parts of a range-separated operator then share
+// screening, primitives, densities and the additions into K (range-separated K
+// of 16 waters def2-TZVP 131 -> 97 ms).  DUAL: the kernel may be given a second
+// part; the per-lane kernels with J are not: a loop around one part kept the
+// compiler from scheduling across it ((pp|ss) 150 -> 168 us, (ss|ss) 246 -> 275
+// of 8 waters def2-SVP), and there two launches serve.
+template <bool DUAL>
+struct Oper {
+    double omega2, full;
+    __device__ __forceinline__ explicit Oper(const JKBuildArgs &a)
+        : omega2(a.omega * a.omega), full(DUAL ? a.full : 0.) {}
+    __device__ __forceinline__ int parts() const { return DUAL && full != 0. ? 2 : 1; }
+};
+
 // One quartet per lane in arithmetic type T (double or float): returns the
 // rows I0 <= i < I1 of the Cartesian block (times the symmetry and
 // normalisation prefactors) in gout[(((i-I0)*nfj+j)*nfk+k)*nfl+l].
 // pij: the primitives of the (uniform) ij pair; pkl: records of this lane's kl
 // pair.  `loaded` is called once, when the first kl record has arrived.
 template <int LI, int LJ, int LK, int LL, typename T, int I0 = 0, int I1 = ncart(LI),
-          typename Pij, typename F>
+          bool DUAL = false, typename Pij, typename F>
 __device__ __forceinline__ void eri_lane(T *gout, const Pij &pij, int nij,
                                          const double *pkl, int nkl, const double *rij,
                                          const double *rk, const double *rkl,
                                          const JKRysTable &rys, const lds_double *rows,
-                                         double fac_sym, double omega2, F &&loaded)
+                                         double fac_sym, const Oper<DUAL> &op, F &&loaded)
 {
     constexpr int NFJ = ncart(LJ), NFK = ncart(LK), NFL = ncart(LL);
     constexpr int NF = (I1 - I0) * NFJ * NFK * NFL;
@@ -1140,55 +1156,64 @@ __device__ __forceinline__ void eri_lane(T *gout, const Pij &pij, int nij,
             T r_aa = rcp64(aij + akl);
             T theta = aij * akl * r_aa;
             T fac = (T)K_d * Kkl * rsqrt64(aij + akl);
-            T rt[N], wt[N];
-            // long-range attenuation erf(omega r)/r: the rule at x a with the
-            // roots scaled by a and the weights by sqrt(a)
-            T aw = (T)1;
-            if (omega2 > 0.) aw = (T)omega2 / ((T)omega2 + theta);
-            if constexpr (sizeof(T) == sizeof(float) && N <= 3) {
-                // the rule of the Boys moments in FP64 is cheaper than the float
-                // Chebyshev series for up to three roots
-                double rd[N], wd[N];
-                rys_roots<N>(rys, rows, (double)(theta * rr * aw), rd, wd);
+            auto add_part = [&](double omega2, T fac) {
+                T rt[N], wt[N];
+                // long-range attenuation erf(omega r)/r: the rule at x a with the
+                // roots scaled by a and the weights by sqrt(a)
+                T aw = (T)1;
+                if (omega2 > 0.) aw = (T)omega2 / ((T)omega2 + theta);
+                if constexpr (sizeof(T) == sizeof(float) && N <= 3) {
+                    // the rule of the Boys moments in FP64 is cheaper than the float
+                    // Chebyshev series for up to three roots
+                    double rd[N], wd[N];
+                    rys_roots<N>(rys, rows, (double)(theta * rr * aw), rd, wd);
 #pragma unroll
-                for (int i = 0; i < N; ++i) { rt[i] = (T)rd[i]; wt[i] = (T)wd[i]; }
-            } else {
-                rys_roots<N>(rys, rows, theta * rr * aw, rt, wt);
-            }
-            if (omega2 > 0.) {
-                const T sa = sqrt(aw);
-#pragma unroll
-                for (int i = 0; i < N; ++i) { rt[i] *= aw; wt[i] *= sa; }
-            }
-#pragma unroll
-            for (int ir = 0; ir < N; ++ir) {
-                T rt_aa = rt[ir] * r_aa;
-                T rt_aij = rt_aa * akl, rt_akl = rt_aa * aij;
-                T b10 = (T).5 * raij * ((T)1 - rt_aij);
-                T b01 = (T).5 * rakl * ((T)1 - rt_akl);
-                T b00 = (T).5 * rt_aa;
-                T gx[GS], gy[GS], gz[GS];
-                build_g<LI, LJ, LK, LL>(gx, (T)1, PA[0] - rt_aij * PQ[0], QC[0] + rt_akl * PQ[0],
-                                        b10, b01, b00, rij_t[0], rkl_t[0]);
-                build_g<LI, LJ, LK, LL>(gy, (T)1, PA[1] - rt_aij * PQ[1], QC[1] + rt_akl * PQ[1],
-                                        b10, b01, b00, rij_t[1], rkl_t[1]);
-                build_g<LI, LJ, LK, LL>(gz, wt[ir] * fac, PA[2] - rt_aij * PQ[2],
-                                        QC[2] + rt_akl * PQ[2], b10, b01, b00, rij_t[2], rkl_t[2]);
-#pragma unroll
-                for (int i = I0; i < I1; ++i)
-#pragma unroll
-                for (int j = 0; j < NFJ; ++j)
-#pragma unroll
-                for (int k = 0; k < NFK; ++k)
-#pragma unroll
-                for (int l = 0; l < NFL; ++l) {
-                    constexpr int SJ = LL+1, SK = (LK+1)*(LL+1), SI = (LJ+1)*(LK+1)*(LL+1);
-                    int ix = ci.x[i]*SI + cj.x[j]*SK + ck.x[k]*SJ + cl.x[l];
-                    int iy = ci.y[i]*SI + cj.y[j]*SK + ck.y[k]*SJ + cl.y[l];
-                    int iz = ci.z[i]*SI + cj.z[j]*SK + ck.z[k]*SJ + cl.z[l];
-                    int n = (((i - I0)*NFJ + j)*NFK + k)*NFL + l;
-                    gout[n] = fma(gx[ix] * gy[iy], gz[iz], gout[n]);
+                    for (int i = 0; i < N; ++i) { rt[i] = (T)rd[i]; wt[i] = (T)wd[i]; }
+                } else {
+                    rys_roots<N>(rys, rows, theta * rr * aw, rt, wt);
                 }
+                if (omega2 > 0.) {
+                    const T sa = sqrt(aw);
+#pragma unroll
+                    for (int i = 0; i < N; ++i) { rt[i] *= aw; wt[i] *= sa; }
+                }
+#pragma unroll
+                for (int ir = 0; ir < N; ++ir) {
+                    T rt_aa = rt[ir] * r_aa;
+                    T rt_aij = rt_aa * akl, rt_akl = rt_aa * aij;
+                    T b10 = (T).5 * raij * ((T)1 - rt_aij);
+                    T b01 = (T).5 * rakl * ((T)1 - rt_akl);
+                    T b00 = (T).5 * rt_aa;
+                    T gx[GS], gy[GS], gz[GS];
+                    build_g<LI, LJ, LK, LL>(gx, (T)1, PA[0] - rt_aij * PQ[0], QC[0] + rt_akl * PQ[0],
+                                            b10, b01, b00, rij_t[0], rkl_t[0]);
+                    build_g<LI, LJ, LK, LL>(gy, (T)1, PA[1] - rt_aij * PQ[1], QC[1] + rt_akl * PQ[1],
+                                            b10, b01, b00, rij_t[1], rkl_t[1]);
+                    build_g<LI, LJ, LK, LL>(gz, wt[ir] * fac, PA[2] - rt_aij * PQ[2],
+                                            QC[2] + rt_akl * PQ[2], b10, b01, b00, rij_t[2], rkl_t[2]);
+#pragma unroll
+                    for (int i = I0; i < I1; ++i)
+#pragma unroll
+                    for (int j = 0; j < NFJ; ++j)
+#pragma unroll
+                    for (int k = 0; k < NFK; ++k)
+#pragma unroll
+                    for (int l = 0; l < NFL; ++l) {
+                        constexpr int SJ = LL+1, SK = (LK+1)*(LL+1), SI = (LJ+1)*(LK+1)*(LL+1);
+                        int ix = ci.x[i]*SI + cj.x[j]*SK + ck.x[k]*SJ + cl.x[l];
+                        int iy = ci.y[i]*SI + cj.y[j]*SK + ck.y[k]*SJ + cl.y[l];
+                        int iz = ci.z[i]*SI + cj.z[j]*SK + ck.z[k]*SJ + cl.z[l];
+                        int n = (((i - I0)*NFJ + j)*NFK + k)*NFL + l;
+                        gout[n] = fma(gx[ix] * gy[iy], gz[iz], gout[n]);
+                    }
+                }
+            };
+            if constexpr (DUAL) {
+#pragma unroll 1
+                for (int part = op.parts() - 1; part >= 0; --part)
+                    add_part(part ? 0. : op.omega2, part ? fac * (T)op.full : fac);
+            } else {
+                add_part(op.omega2, fac);
             }
         }
     }
@@ -1305,7 +1330,7 @@ __device__ __forceinline__ void lane_batch(const JKBuildArgs &a, const ShellPair
         eri_lane<LI, LJ, LK, LL, T, I0, I1>(
             gout, PijGlobal{a.pdata_ij + (size_t)pij * nij * PREC, sp.ri}, nij,
             a.pdata_kl + (size_t)pkl * nkl * PREC, nkl, sp.rij, rk3, rkl, a.rys, rows, fac_sym,
-            a.omega * a.omega, [] {});
+            Oper<false>(a), [] {});
         for (int id = 0; id < a.n_dm; ++id) {
             const double *D = a.dm + id * nao2;
             if (a.vk) {
@@ -1648,9 +1673,9 @@ void jk_lane_kernel(JKBuildArgs a, TaskBatch batch)
 // Chunked classes with an f shell stay on jk_lane_kernel: the J_kl block held
 // over the chunks costs them more registers than the waits ((fp|fs) 20.8 -> 22.5,
 // (fp|pp) 33.7 -> 34.5, (fp|ds) 29.4 -> 29.9).
-template <int LI, int LJ, int LK, int LL>
+template <int LI, int LJ, int LK, int LL, bool WJ>
 struct LaneFast {
-    static constexpr bool ON = LI < 3 || LaneChunk<LI, LJ, LK, LL>::NCH == 1;
+    static constexpr bool ON = !WJ || LI < 3 || LaneChunk<LI, LJ, LK, LL>::NCH == 1;
 };
 
 struct ItemLds {
@@ -1692,9 +1717,9 @@ __device__ __forceinline__ void lane_batch_fast(const JKBuildArgs &a, const Shel
         constexpr int I1 = I0 + CH < NFI ? I0 + CH : NFI;
         constexpr int NI = I1 - I0;
         double gout[NI * NFJ * NFK * NFL];
-        eri_lane<LI, LJ, LK, LL, double, I0, I1>(
+        eri_lane<LI, LJ, LK, LL, double, I0, I1, !WJ>(
             gout, PijLds{it.pij}, nij, a.pdata_kl + (size_t)pkl * nkl * PREC, nkl, sp.rij, rk3,
-            rkl, a.rys, it.rows, fac_sym, a.omega * a.omega, [&] {
+            rkl, a.rys, it.rows, fac_sym, Oper<!WJ>(a), [&] {
                 if constexpr (WJ && I0 == 0) {
                     // J_kl of the previous batch
                     if (pend_off != ~0u) {
@@ -2105,7 +2130,7 @@ void jk_team_kernel(JKBuildArgs a, TaskBatch batch)
             if (bas_ij == bas_kl) fac_sym *= .5;
             const double *rk = a.env + a.bas[ksh * 8 + 7], *rl = a.env + a.bas[lsh * 8 + 7];
             double rkl[3] = {rl[0] - rk[0], rl[1] - rk[1], rl[2] - rk[2]};
-            const double omega2 = a.omega * a.omega;
+            const Oper<true> op(a);
             const int nij = a.iprim * a.jprim, nkl = a.kprim * a.lprim;
             const double *pdij = a.pdata_ij + (size_t)wi.pij * nij * PREC;
             const double *pdkl = a.pdata_kl + (size_t)pkl * nkl * PREC;
@@ -2133,81 +2158,85 @@ void jk_team_kernel(JKBuildArgs a, TaskBatch batch)
                 theta = aij * akl * r_aa;
                 fac = pr[5] * qr[5] * fac_sym * sqrt(r_aa);
             };
-            for (int pq0 = 0; pq0 < npq; pq0 += PB) {
-                const int np = min(PB, npq - pq0);
-                __syncthreads();
-                // roots: lane (p, r) for p < np, r < N
-                if (active && tl < np * N) {
-                    const int p = tl / N, r = tl - p * N;
-                    double aij, raij, akl, rakl, PA[3], PQ[3], QC[3], r_aa, theta, rr, fac;
-                    prim(pq0 + p, aij, raij, akl, rakl, PA, PQ, QC, r_aa, theta, rr, fac);
-                    double rt, wt;
-                    if (omega2 > 0.) {
-                        // long-range attenuation (see eri_lane)
-                        const double aw = omega2 / (omega2 + theta);
-                        rys_root_one<N>(a.rys, theta * rr * aw, r, rt, wt);
-                        rt *= aw; wt *= sqrt(aw);
-                    } else {
-                        rys_root_one<N>(a.rys, theta * rr, r, rt, wt);
+#pragma unroll 1
+            for (int part = op.parts() - 1; part >= 0; --part) {
+            const double omega2 = part ? 0. : op.omega2;
+                for (int pq0 = 0; pq0 < npq; pq0 += PB) {
+                    const int np = min(PB, npq - pq0);
+                    __syncthreads();
+                    // roots: lane (p, r) for p < np, r < N
+                    if (active && tl < np * N) {
+                        const int p = tl / N, r = tl - p * N;
+                        double aij, raij, akl, rakl, PA[3], PQ[3], QC[3], r_aa, theta, rr, fac;
+                        prim(pq0 + p, aij, raij, akl, rakl, PA, PQ, QC, r_aa, theta, rr, fac);
+                        double rt, wt;
+                        if (omega2 > 0.) {
+                            // long-range attenuation (see eri_lane)
+                            const double aw = omega2 / (omega2 + theta);
+                            rys_root_one<N>(a.rys, theta * rr * aw, r, rt, wt);
+                            rt *= aw; wt *= sqrt(aw);
+                        } else {
+                            rys_root_one<N>(a.rys, theta * rr, r, rt, wt);
+                        }
+                        double *rw = my + p * S::G_DBL;
+                        rw[2*r] = rt; rw[2*r+1] = wt;
                     }
-                    double *rw = my + p * S::G_DBL;
-                    rw[2*r] = rt; rw[2*r+1] = wt;
-                }
-                __syncthreads();
-                // 2D tables: lane (p, r, d) for p < np
-                if (active && tl < np * 3 * N) {
-                    const int p = tl / (3 * N), rd = tl - p * (3 * N);
-                    const int r = rd / 3, d = rd - (rd / 3) * 3;
-                    double aij, raij, akl, rakl, PA[3], PQ[3], QC[3], r_aa, theta, rr, fac;
-                    prim(pq0 + p, aij, raij, akl, rakl, PA, PQ, QC, r_aa, theta, rr, fac);
-                    const double *rw = my + p * S::G_DBL;
-                    double rt_aa = rw[2*r] * r_aa;
-                    double rt_aij = rt_aa * akl, rt_akl = rt_aa * aij;
-                    double b10 = .5 * raij * (1. - rt_aij);
-                    double b01 = .5 * rakl * (1. - rt_akl);
-                    double b00 = .5 * rt_aa;
-                    double g[GS];
-                    double pa = d == 0 ? PA[0] : (d == 1 ? PA[1] : PA[2]);
-                    double pq = d == 0 ? PQ[0] : (d == 1 ? PQ[1] : PQ[2]);
-                    double qc = d == 0 ? QC[0] : (d == 1 ? QC[1] : QC[2]);
-                    double rd_ = d == 0 ? sp.rij[0] : (d == 1 ? sp.rij[1] : sp.rij[2]);
-                    double kd = d == 0 ? rkl[0] : (d == 1 ? rkl[1] : rkl[2]);
-                    double g00 = d == 2 ? rw[2*r+1] * fac : 1.;
-                    build_g<LI, LJ, LK, LL, double>(g, g00, pa - rt_aij * pq,
-                                            qc + rt_akl * pq,
-                                            b10, b01, b00, rd_, kd);
-                    double *dst = my + p * S::G_DBL + 2 * N + (r * 3 + d) * GS;
+                    __syncthreads();
+                    // 2D tables: lane (p, r, d) for p < np
+                    if (active && tl < np * 3 * N) {
+                        const int p = tl / (3 * N), rd = tl - p * (3 * N);
+                        const int r = rd / 3, d = rd - (rd / 3) * 3;
+                        double aij, raij, akl, rakl, PA[3], PQ[3], QC[3], r_aa, theta, rr, fac;
+                        prim(pq0 + p, aij, raij, akl, rakl, PA, PQ, QC, r_aa, theta, rr, fac);
+                        const double *rw = my + p * S::G_DBL;
+                        double rt_aa = rw[2*r] * r_aa;
+                        double rt_aij = rt_aa * akl, rt_akl = rt_aa * aij;
+                        double b10 = .5 * raij * (1. - rt_aij);
+                        double b01 = .5 * rakl * (1. - rt_akl);
+                        double b00 = .5 * rt_aa;
+                        double g[GS];
+                        double pa = d == 0 ? PA[0] : (d == 1 ? PA[1] : PA[2]);
+                        double pq = d == 0 ? PQ[0] : (d == 1 ? PQ[1] : PQ[2]);
+                        double qc = d == 0 ? QC[0] : (d == 1 ? QC[1] : QC[2]);
+                        double rd_ = d == 0 ? sp.rij[0] : (d == 1 ? sp.rij[1] : sp.rij[2]);
+                        double kd = d == 0 ? rkl[0] : (d == 1 ? rkl[1] : rkl[2]);
+                        double g00 = d == 2 ? rw[2*r+1] * (part ? fac * op.full : fac) : 1.;
+                        build_g<LI, LJ, LK, LL, double>(g, g00, pa - rt_aij * pq,
+                                                qc + rt_akl * pq,
+                                                b10, b01, b00, rd_, kd);
+                        double *dst = my + p * S::G_DBL + 2 * N + (r * 3 + d) * GS;
 #pragma unroll
-                    for (int n = 0; n < GS; ++n) dst[n] = g[n];
-                }
-                __syncthreads();
-                if (active && has_row) {
-                    int ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0;
-                    // Cartesian powers of this row's i and j (runtime lookup)
+                        for (int n = 0; n < GS; ++n) dst[n] = g[n];
+                    }
+                    __syncthreads();
+                    if (active && has_row) {
+                        int ax = 0, ay = 0, az = 0, bx = 0, by = 0, bz = 0;
+                        // Cartesian powers of this row's i and j (runtime lookup)
 #pragma unroll
-                    for (int i = 0; i < NFI; ++i)
-                        if (i == irow) { ax = ci.x[i]; ay = ci.y[i]; az = ci.z[i]; }
+                        for (int i = 0; i < NFI; ++i)
+                            if (i == irow) { ax = ci.x[i]; ay = ci.y[i]; az = ci.z[i]; }
 #pragma unroll
-                    for (int j = 0; j < NFJ; ++j)
-                        if (j == jrow) { bx = cj.x[j]; by = cj.y[j]; bz = cj.z[j]; }
-                    const int ox = ax * SI + bx * SK, oy = ay * SI + by * SK, oz = az * SI + bz * SK;
-                    for (int p = 0; p < np; ++p) {
-                        const double *gb = my + p * S::G_DBL + 2 * N;
-                        for (int r = 0; r < N; ++r) {
-                            const double *gx = gb + (r * 3 + 0) * GS + ox;
-                            const double *gy = gb + (r * 3 + 1) * GS + oy;
-                            const double *gz = gb + (r * 3 + 2) * GS + oz;
-                            double sx[SK], sy[SK], sz[SK];
+                        for (int j = 0; j < NFJ; ++j)
+                            if (j == jrow) { bx = cj.x[j]; by = cj.y[j]; bz = cj.z[j]; }
+                        const int ox = ax * SI + bx * SK, oy = ay * SI + by * SK, oz = az * SI + bz * SK;
+                        for (int p = 0; p < np; ++p) {
+                            const double *gb = my + p * S::G_DBL + 2 * N;
+                            for (int r = 0; r < N; ++r) {
+                                const double *gx = gb + (r * 3 + 0) * GS + ox;
+                                const double *gy = gb + (r * 3 + 1) * GS + oy;
+                                const double *gz = gb + (r * 3 + 2) * GS + oz;
+                                double sx[SK], sy[SK], sz[SK];
 #pragma unroll
-                            for (int n = 0; n < SK; ++n) { sx[n] = gx[n]; sy[n] = gy[n]; sz[n] = gz[n]; }
+                                for (int n = 0; n < SK; ++n) { sx[n] = gx[n]; sy[n] = gy[n]; sz[n] = gz[n]; }
 #pragma unroll
-                            for (int k = 0; k < NFK; ++k)
+                                for (int k = 0; k < NFK; ++k)
 #pragma unroll
-                            for (int l = 0; l < NFL; ++l) {
-                                int kx = ck.x[k]*SJ + cl.x[l];
-                                int ky = ck.y[k]*SJ + cl.y[l];
-                                int kz = ck.z[k]*SJ + cl.z[l];
-                                acc[k*NFL + l] = fma(sx[kx] * sy[ky], sz[kz], acc[k*NFL + l]);
+                                for (int l = 0; l < NFL; ++l) {
+                                    int kx = ck.x[k]*SJ + cl.x[l];
+                                    int ky = ck.y[k]*SJ + cl.y[l];
+                                    int kz = ck.z[k]*SJ + cl.z[l];
+                                    acc[k*NFL + l] = fma(sx[kx] * sy[ky], sz[kz], acc[k*NFL + l]);
+                                }
                             }
                         }
                     }
@@ -2418,25 +2447,25 @@ static const ClassInfo *class_info()
         c.cost = T::N * (3. * T::NF + 9. * T::GS) + 200.;
         for (int n = 0; n < JK_KERNELS; ++n) { c.occ[n] = occ[n]; c.fn[n] = nullptr; }
         if constexpr (T::LANE) {
-            constexpr bool FAST = LaneFast<LI, LJ, LK, LL>::ON;
+            constexpr bool FAST_J = LaneFast<LI, LJ, LK, LL, true>::ON;
             c.fn[0] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 0, 2>;
             c.fn[1] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 2>;
-            if constexpr (FAST) {
+            if constexpr (FAST_J) {
                 c.fn[2] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2, 1>;
                 c.fn[3] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2, 1>;
-                c.fn[4] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 1>;
                 c.fn[8] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 2, 2>;
                 c.fn[9] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, false, 2, 2>;
-                c.fn[10] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 2>;
             }
+            c.fn[4] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 1>;
+            c.fn[10] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 2, 2>;
             if constexpr (FourWaves<LI, LJ, LK, LL>::ON) {
                 c.fn[5] = (const void *)jk_lane_kernel<LI, LJ, LK, LL, 1, 4>;
-                if constexpr (FAST) {
+                if constexpr (FAST_J) {
                     c.fn[6] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4, 1>;
-                    c.fn[7] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 1>;
                     c.fn[11] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, true, true, 4, 2>;
-                    c.fn[12] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 2>;
                 }
+                c.fn[7] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 1>;
+                c.fn[12] = (const void *)jk_lane_fast_kernel<LI, LJ, LK, LL, false, true, 4, 2>;
             }
             for (int n = 0; n < JK_KERNELS; ++n) {
                 const int nw = lane_waves(n), nd = lane_densities(n);

@@ -310,6 +310,10 @@ static int check_args(const JKBuildArgs *args, JKBuildArgs &a, const char *who)
     }
     if (!table_ok(a.rys)) { set_err("%s: Rys table not set", who); return 3; }
     if (!(a.omega >= 0.)) { set_err("%s: omega must be >= 0 (erf attenuation)", who); return 3; }
+    if (a.full != 0. && !(a.omega > 0.)) {
+        set_err("%s: a full-range part goes with an attenuated one only", who);
+        return 3;
+    }
     for (int t = 0; t < 2; ++t) {
         const JKWindows &w = a.kl_win[t];
         if (w.win && (w.n_win <= 0 || w.width <= 0 || !w.pairs || !w.q || !w.pdata)) {
@@ -380,6 +384,10 @@ static int check_ip1(const JKBuildArgs *args, JKBuildArgs &a, const double *ejk)
 {
     const int st = check_args(args, a, "jk_energy_ip1");
     if (st) return st;
+    if (a.full != 0.) {
+        set_err("jk_energy_ip1: full is for J/K builds only");
+        return 3;
+    }
     if (a.swap_ijkl) {
         set_err("jk_energy_ip1: swap_ijkl is for J/K builds only");
         return 3;

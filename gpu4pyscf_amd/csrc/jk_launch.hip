@@ -229,6 +229,9 @@ static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
 struct Kernel {
     const void *fn;
     int threads;
+    // 0 the whole operator; 1 and 2 its attenuated and its full-range part, for
+    // the kernels that take one at a time (runtime l; per-lane ones with J)
+    int part;
 };
 
 struct Launch {
@@ -293,9 +296,9 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
     std::vector<int> order;
     auto add = [&](int key, const Kernel &kern, const Item &it) {
         if (it.blocks > INT_MAX) return false;
-        Group &g = by_kernel[key];
+        Group &g = by_kernel[3 * key + kern.part];
         if (g.items.empty()) {
-            order.push_back(key);
+            order.push_back(3 * key + kern.part);
             g.k = kern;
         }
         g.items.push_back(it);
@@ -325,7 +328,7 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
         const void *ip1 = run.mode != GEN_JK && small ? jk_ip1_lane_kernel_of(key) : nullptr;
         Kernel kern;
         if (ip1) {
-            kern = {ip1, WAVE};
+            kern = {ip1, WAVE, 0};
             const int nchunks = std::min((IP1_ITEMS + k.npairs_ij - 1) / k.npairs_ij,
                                          (k.npairs_kl + WAVE - 1) / WAVE);
             d.kl_chunk = (k.npairs_kl + nchunks - 1) / nchunks;
@@ -335,14 +338,15 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
             it.cost = quartets * ncart(k.li) * ncart(k.lj) * ncart(k.lk) * ncart(k.ll);
         } else if (run.mode != GEN_JK || !small) {
             key = -1;
-            kern = {jk_generic_kernel_of(run.mode), GEN_TB};
+            kern = {jk_generic_kernel_of(run.mode), GEN_TB, 0};
             if (!jk_generic_plan(k, run.mode, d, it.blocks, it.lds)) return hipErrorNotSupported;
             it.per_cu = (int)(lim.lds_cu / (it.lds + 4096));
             it.cost = quartets * ncart(k.li) * ncart(k.lj) * ncart(k.lk) * ncart(k.ll);
+            if (run.mode == GEN_JK && a.full != 0.) kern.part = 1;
         } else {
             const ClassInfo *c = class_info_of(key);
             if (!c) return hipErrorNotSupported;
-            it.cost = quartets * c->cost;
+            it.cost = quartets * c->cost * (a.full != 0. ? 2 : 1);
             if (c->lane) {
                 // the fast kernels in as many launches as the densities take
                 for (int dm0 = 0; dm0 < a.n_dm;) {
@@ -350,17 +354,23 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
                     const int f = plan_lane(a, k, *c, pm, a.n_dm - dm0, lim, part);
                     const int nd = lane_densities(f);
                     if (nd) part.d.ls_swap |= (uint32_t)dm0 << 17;
-                    if (!add(key * JK_KERNELS + f, {c->fn[f], c->threads[f]}, part))
-                        return hipErrorInvalidConfiguration;
+                    const bool split = a.full != 0. && !(nd && !a.vj);
+                    for (int p = split ? 1 : 0; p <= (split ? 2 : 0); ++p)
+                        if (!add(key * JK_KERNELS + f, {c->fn[f], c->threads[f], p}, part))
+                            return hipErrorInvalidConfiguration;
                     dm0 += nd ? nd : a.n_dm;
                 }
                 continue;
             }
             plan_team(a, k, *c, lim, it);
-            kern = {c->fn[pm], c->threads[pm]};
+            kern = {c->fn[pm], c->threads[pm], 0};
             key = key * JK_KERNELS + pm;
         }
         if (!add(key, kern, it)) return hipErrorInvalidConfiguration;
+        if (kern.part == 1) {
+            kern.part = 2;
+            if (!add(key, kern, it)) return hipErrorInvalidConfiguration;
+        }
     }
     std::vector<Launch> launches;
     for (int key : order)
@@ -372,7 +382,14 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
     for (Launch &l : launches) {
         const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
         load[s] += l.cost;
-        void *args[] = {(void *)&a, &l.b, (void *)&run.ex};
+        JKBuildArgs p = a;
+        if (l.k.part) p.full = 0.;
+        if (l.k.part == 2) {
+            p.scale = a.scale * a.full;
+            p.omega = 0.;
+            p.n_quartets = p.n_quartets_fp32 = p.quartet_hash = nullptr;
+        }
+        void *args[] = {&p, &l.b, (void *)&run.ex};
         const hipError_t err = hipLaunchKernel(l.k.fn, dim3((unsigned)l.blocks),
                                                dim3(l.k.threads), args, l.lds,
                                                (hipStream_t)streams[s]);

@@ -14,7 +14,7 @@ _here = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_here, 'libjkhip.so')
 TABLE_PATH = os.path.join(os.path.dirname(_here), 'csrc', 'rys_table.npz')
 
-JK_ABI_VERSION = 14
+JK_ABI_VERSION = 15
 JK_RYS_NMAX = 11
 JK_BOYS_M = 14
 JK_LMAX = 5
@@ -79,6 +79,7 @@ class JKBuildArgs(ctypes.Structure):
         ('repl_stride', ctypes.c_int64),
         ('omega', ctypes.c_double),
         ('scale', ctypes.c_double),
+        ('full', ctypes.c_double),
         ('screen', ctypes.c_int),
         ('kl_win', JKWindows * 2),
         ('kl_win_policy', ctypes.c_int),

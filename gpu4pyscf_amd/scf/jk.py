@@ -549,9 +549,8 @@ class _VHFOpt:
         fp32_tol: evaluate in FP32 the quartets whose bound
         sqrt|(ij|ij)| sqrt|(kl|kl)| max|D| is below fp32_tol (None: all FP64).
         omega, lr_factor, sr_factor: the operator of K (default: the
-        molecule's omega); a range-separated operator takes two launches of
-        every class task (full range and erf-attenuated), whose counters are
-        those of the first.  J always uses the molecule's operator; when K's
+        molecule's omega); the two parts (full range and erf-attenuated) of a
+        range-separated operator share the quartets.  J always uses the molecule's operator; when K's
         differs, J comes from a J-only build and K from a K-only build, as in
         gpu4pyscf/scf/jk.py:129-135 (the counters are then the K build's).
         screen: the density blocks of the survival test, 'jk' (all six, the
@@ -633,15 +632,18 @@ class _VHFOpt:
         args.repl_stride = dms.numel()
         args.screen = clib.JK_SCREEN[screen]
         args.kl_win_policy = int(self.kl_win_policy)
-        # launch passes of the operator: (omega, scale, with J, with K)
-        runs = [(w, f, with_j, with_k)
-                for w, f in self.operator_passes(omega, lr_factor, sr_factor)]
+        # launch passes of the operator: (omega, scale, full-range part), one
+        # unless its parts are of very different size
+        runs = [(w, f, 0.) for w, f in self.operator_passes(omega, lr_factor, sr_factor)]
+        if len(runs) == 2 and 1e-6 < abs(runs[0][1] / runs[1][1]) < 1e6:
+            runs = [(runs[1][0], runs[1][1], runs[0][1] / runs[1][1])]
         with self.fork_streams(dms.device) as streams:
-            for n_run, (w, f, rj, rk) in enumerate(runs):
+            for n_run, (w, f, full) in enumerate(runs):
                 args.omega = w
                 args.scale = f
-                args.vj = vj.data_ptr() if rj else None
-                args.vk = vk.data_ptr() if rk else None
+                args.full = full
+                args.vj = vj.data_ptr() if with_j else None
+                args.vk = vk.data_ptr() if with_k else None
                 first = n_run == 0
                 # one native call; with per-launch timing a launch per task,
                 # from the last (f classes, the longest) to the first

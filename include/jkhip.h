@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define JK_ABI_VERSION  14
+#define JK_ABI_VERSION  15
 #define JK_RYS_NMAX     11      /* max Rys roots: (hh|hh) */
 #define JK_LMAX         5       /* max angular momentum on the GPU path */
 
@@ -124,11 +124,13 @@ typedef struct {
     /* Operator: scale * erf(omega r)/r for omega > 0, scale / r for
      * omega == 0 (scale multiplies every integral of the launch).  The
      * range-separated operators of gpu4pyscf/scf/jk.py:1122-1168,
-     * lr erf(w r)/r + sr erfc(w r)/r = sr / r + (lr - sr) erf(w r)/r, are
-     * built from two launches of each class task; the reference instead
-     * doubles the Rys roots (rys_roots_for_k.cu:19-68). */
+     * lr erf(w r)/r + sr erfc(w r)/r = sr / r + (lr - sr) erf(w r)/r, take
+     * full: scale * (erf(omega r)/r + full / r) for omega > 0 (0 for the other
+     * operators, and for jk_energy_ip1); a second set of Rys roots per primitive
+     * quartet, as in the reference (rys_roots_for_k.cu:19-68). */
     double omega;
     double scale;           /* 0 is taken as 1 */
+    double full;
     /* Survival screen: which density blocks keep a quartet whose bound
      * q_ij + q_kl + dm_cond exceeds the cutoff.  JK_SCREEN_JK: any of the
      * six blocks D_ij, D_kl, D_ik, D_jk, D_il, D_jl (RYS_build_jk,

@@ -175,3 +175,28 @@ def test_energy_gradient_tzvp_golden():
     assert abs(ejk.sum()) < 1e-9
     assert abs(O.fp(ejk) - 2710.490337642) < 1e-9
     assert abs(ejk - ref).max() < 1e-10 * max(1., abs(ref).max())
+
+
+@pytest.mark.parametrize('basis', ['def2-tzvp', ('def2-svp', [[4, [.9, 1.]]])])
+@pytest.mark.parametrize('n_dm', [1, 2, 3])
+@pytest.mark.parametrize('with_j', [False, True])
+def test_operator_parts_together_match_their_sum(basis, n_dm, with_j):
+    """lr erf + sr erfc in one build (two sets of roots per quartet, or two
+    launches) against full range and erf in builds of their own, on one screen:
+    the same terms in another order, up to 1e4 of them per element."""
+    import torch
+    from gpu4pyscf_amd.gto import geometry as G
+    from gpu4pyscf_amd.gto.mole import M
+    from gpu4pyscf_amd.scf import jk
+    mol = M(atom=G.to_string(G.water_cluster((2, 1, 1), 3., seed=4)), basis=basis)
+    opt = jk._VHFOpt(mol).build()
+    dm = np.random.default_rng(8).standard_normal((n_dm, mol.nao, mol.nao))
+    dm = opt.apply_coeff_C_mat_CT(torch.as_tensor(dm + dm.transpose(0, 2, 1), device='cuda'))
+    kw = dict(with_j=with_j, screen='jk' if with_j else 'k', omega=.3)
+    got = opt.get_jk(dm, 1, lr_factor=.65, sr_factor=.2, **kw)
+    full = opt.get_jk(dm, 1, lr_factor=1., sr_factor=1., **kw)
+    erf = opt.get_jk(dm, 1, lr_factor=1., sr_factor=0., **kw)
+    for x, y, z in zip(got, full, erf):
+        if x is not None:
+            ref = .2 * y + .45 * z
+            assert float((x - ref).abs().max()) <= 1e4 * 2.2e-16 * float(y.abs().max())
