@@ -121,6 +121,7 @@ class _VHFOpt(jk_mod._VHFOpt):
         rows, bm, step = self._boys_meta
         dm_cond = torch.empty((nbas, nbas), dtype=torch.float32, device=dev)
         work = torch.empty((nbas, nbas), dtype=torch.float64, device=dev)
+        vj_rys = None
         for n in range(dms.shape[0]):
             dm = dms[n]
             clib.check(lib.jk_dm_cond(ptr(dm_cond), ptr(work), ptr(dm), 1, nao,
@@ -153,16 +154,33 @@ class _VHFOpt(jk_mod._VHFOpt):
             args.dm_penalty = dm_penalty
             # the molecule's operator (screening q_cond uses the same)
             args.omega = float(getattr(self.mol, 'omega', 0.) or 0.)
-            for a, b in self._md_tasks:
-                args.lij, args.lkl = sum(self._md_l[a]), sum(self._md_l[b])
-                args.npairs_ij, args.npairs_kl = len(d['pairs'][a]), len(d['pairs'][b])
-                args.pdata_ij, args.pdata_kl = d['pdata'][a].data_ptr(), d['pdata'][b].data_ptr()
-                args.q_ij, args.q_kl = d['q'][a].data_ptr(), d['q'][b].data_ptr()
-                args.dmax_ij, args.dmax_kl = dmax[a].data_ptr(), dmax[b].data_ptr()
-                args.pairs_ij, args.pairs_kl = d['pairs'][a].data_ptr(), d['pairs'][b].data_ptr()
-                args.dh_kl = dh[b].data_ptr()
-                args.jh_ij = jh[a].data_ptr()
-                clib.check(lib.jk_md_build_j(ctypes.byref(args), stream), 'jk_md_build_j')
+            # the tasks over the side streams, each on the one with the least work
+            # so far; the Rys build beside the last density's reads a maximum of
+            # its own on the caller's stream before it launches, and must not wait
+            # for them (16 waters def2-TZVP: 47.9 ms one after the other)
+            with self.fork_streams(dev) as streams:
+                side = streams[1:] or streams
+                load = [0.] * len(side)
+                for a, b in self._md_tasks:
+                    args.lij, args.lkl = sum(self._md_l[a]), sum(self._md_l[b])
+                    args.npairs_ij, args.npairs_kl = len(d['pairs'][a]), len(d['pairs'][b])
+                    args.pdata_ij = d['pdata'][a].data_ptr()
+                    args.pdata_kl = d['pdata'][b].data_ptr()
+                    args.q_ij, args.q_kl = d['q'][a].data_ptr(), d['q'][b].data_ptr()
+                    args.dmax_ij, args.dmax_kl = dmax[a].data_ptr(), dmax[b].data_ptr()
+                    args.pairs_ij = d['pairs'][a].data_ptr()
+                    args.pairs_kl = d['pairs'][b].data_ptr()
+                    args.dh_kl = dh[b].data_ptr()
+                    args.jh_ij = jh[a].data_ptr()
+                    s = load.index(min(load))
+                    load[s] += (float(args.npairs_ij) * args.npairs_kl *
+                                (_nh(args.lij) * _nh(args.lkl) + 60))
+                    clib.check(lib.jk_md_build_j(ctypes.byref(args),
+                                                 ctypes.c_void_p(side[s].cuda_stream)),
+                               'jk_md_build_j')
+                if n == dms.shape[0] - 1 and self.tasks():
+                    # classes above MD_LMAX: Rys J-only build on the same pair lists
+                    vj_rys = super().get_jk(dms, 1, with_k=False, screen='j')[0]
             for key in self._md_keys:
                 li, lj = self._md_l[key]
                 pairs = d['pairs'][key]
@@ -170,9 +188,7 @@ class _VHFOpt(jk_mod._VHFOpt):
                     ptr(vj[n]), ptr(jh[key]), nao, ptr(pairs), len(pairs),
                     ptr(d['pdata'][key]), li, lj, ptr(d['bas']), ptr(d['env']),
                     ptr(d['ao_loc']), nbas, stream), 'jk_md_hermite_to_j')
-        if self.tasks():
-            # classes above MD_LMAX: Rys J-only build on the same pair lists
-            vj_rys = super().get_jk(dms, 1, with_k=False, screen='j')[0]
+        if vj_rys is not None:
             vj += vj_rys
         if counter is not None:
             c = counter.cpu().numpy()
