@@ -277,6 +277,24 @@ static bool table_has(const JKRysTable &t, int n)
                      t.xmax[n-1] <= (moment_rows(n) - .5) * MOMENT_STEP);
 }
 
+// status of f(), a planning or launching function
+template <typename F>
+static int guarded(const char *who, F &&f)
+{
+    hipError_t err;
+    try {
+        err = f();
+    } catch (const std::bad_alloc &) {
+        set_err("%s: out of host memory", who);
+        return 4;
+    }
+    if (err != hipSuccess) {
+        set_err("%s: %s", who, hipGetErrorString(err));
+        return 4;
+    }
+    return 0;
+}
+
 extern "C" {
 
 const char *jk_last_error(void) { return g_err; }
@@ -417,18 +435,7 @@ static JKRun ip1_run(double *ejk, double j_factor, double k_factor, int n_dm)
 static int launch(const char *who, const JKBuildArgs &a, const JKTask *tasks, int ntasks,
                   void *const *streams, int nstreams, const JKRun &run)
 {
-    hipError_t err;
-    try {
-        err = jk_launch_tasks(a, tasks, ntasks, streams, nstreams, run);
-    } catch (const std::bad_alloc &) {
-        set_err("%s: out of host memory", who);
-        return 4;
-    }
-    if (err != hipSuccess) {
-        set_err("%s: %s", who, hipGetErrorString(err));
-        return 4;
-    }
-    return 0;
+    return guarded(who, [&] { return jk_launch_tasks(a, tasks, ntasks, streams, nstreams, run); });
 }
 
 int jk_build(const JKBuildArgs *args, void *stream)
@@ -444,6 +451,21 @@ int jk_build(const JKBuildArgs *args, void *stream)
     return launch(who, a, &k, 1, &stream, 1, JKRun{GEN_JK, {nullptr, 0., 0.}});
 }
 
+// Validation of every task of a call, from the last to the first; a: the fields
+// they share.
+static int check_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks, bool gradient,
+                       const double *ejk, JKBuildArgs &a)
+{
+    JKBuildArgs in = *args;
+    a = *args;
+    for (int t = ntasks - 1; t >= 0; --t) {
+        set_task(in, tasks[t]);
+        const int st = gradient ? check_ip1(&in, a, ejk) : check_build(&in, a);
+        if (st > 0) return st;
+    }
+    return 0;
+}
+
 int jk_build_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks,
                    void *const *streams, int nstreams)
 {
@@ -452,12 +474,9 @@ int jk_build_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks,
         set_err("jk_build_tasks: null pointer or bad count (%d tasks)", ntasks);
         return 1;
     }
-    JKBuildArgs in = *args, a = *args;
-    for (int t = ntasks - 1; t >= 0; --t) {
-        set_task(in, tasks[t]);
-        const int st = check_build(&in, a);
-        if (st > 0) return st;
-    }
+    JKBuildArgs a;
+    const int st = check_tasks(args, tasks, ntasks, false, nullptr, a);
+    if (st) return st;
     return launch("jk_build_tasks", a, tasks, ntasks, streams, nstreams,
                   JKRun{GEN_JK, {nullptr, 0., 0.}});
 }
@@ -487,17 +506,33 @@ int jk_energy_ip1_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks
         set_err("jk_energy_ip1_tasks: null pointer or bad count (%d tasks)", ntasks);
         return 1;
     }
-    JKBuildArgs in = *args, a = *args;
-    for (int t = ntasks - 1; t >= 0; --t) {
-        set_task(in, tasks[t]);
-        const int st = check_ip1(&in, a, ejk);
-        if (st > 0) return st;
-    }
+    JKBuildArgs a;
+    const int st = check_tasks(args, tasks, ntasks, true, ejk, a);
+    if (st) return st;
     a.n_repl = n_copies;
     a.repl_stride = copy_stride;
     a.vj = a.vk = nullptr;
     return launch("jk_energy_ip1_tasks", a, tasks, ntasks, streams, nstreams,
                   ip1_run(ejk, j_factor, k_factor, a.n_dm));
+}
+
+int jk_plan_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks, int gradient,
+                  JKPlanItem *out, int nmax, int *nitems)
+{
+    g_err[0] = 0;
+    if (!args || (ntasks > 0 && !tasks) || ntasks < 0 || !nitems || nmax < 0 || (nmax > 0 && !out)) {
+        set_err("jk_plan_tasks: null pointer or bad count (%d tasks)", ntasks);
+        return 1;
+    }
+    double none;            // the plan of a gradient needs no result array
+    JKBuildArgs a;
+    const int st = check_tasks(args, tasks, ntasks, gradient != 0, &none, a);
+    if (st) return st;
+    const JKRun run = gradient ? ip1_run(nullptr, 1., 1., a.n_dm) : JKRun{GEN_JK, {nullptr, 0., 0.}};
+    if (gradient) a.vj = a.vk = nullptr;
+    return guarded("jk_plan_tasks", [&] {
+        return jk_plan_launches(a, tasks, ntasks, run, out, nmax, *nitems);
+    });
 }
 
 int jk_pair_data(double *out, const uint32_t *pairs, int npairs, int iprim,

@@ -46,3 +46,8 @@ struct JKRun {
 // Launches `ntasks` validated tasks; a supplies the fields they share.
 hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
                            void *const *streams, int nstreams, const JKRun &run);
+
+// The launches that jk_launch_tasks would make (jk_plan_tasks): the first nmax
+// items into out, their number into n.
+hipError_t jk_plan_launches(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                            const JKRun &run, JKPlanItem *out, int nmax, int &n);

@@ -86,10 +86,10 @@ static int blocks_per_cu(const ClassInfo &c, int f, size_t bytes, const DeviceLi
     return std::max(1, std::min(nb, by_lds));
 }
 
-// One task of a launch.
+// One task, or a run of its ij pairs, in a launch.
 struct Item {
     TaskDesc d;
-    long blocks;
+    long blocks;        // the same number for every ij pair
     size_t lds;
     int per_cu;         // workgroups per CU with this LDS
     double cost;        // rough work of the task
@@ -125,7 +125,7 @@ static bool plan_lane_rows(const JKBuildArgs &a, const JKTask &k, const ClassInf
     // (ps|ps) 55.9 -> 62.4, (ds|ps) 35.1 -> 41.1, (ds|pp) 31.3 -> 36.2)
     const JKWindows &w = k.kl_win[fast && c.nfij * nd >= 9 && k.kl_win[1].win ? 1 : 0];
     const long blocks_w = w.win ? (long)k.npairs_ij * w.n_win : 0;
-    const bool have_win = w.win && blocks_w <= INT_MAX && LANE_KROWS >= 2;
+    const bool have_win = w.win && LANE_KROWS >= 2;
     long best_key = -1;
     for (int win = 0; win < (have_win ? 2 : 1); ++win) {
         const int kn = win ? w.width : k.k_nao, ln = win ? 0 : k.l_nao;
@@ -210,7 +210,7 @@ static void plan_team(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c,
         // enough work items to fill the GPU
         const size_t bytes = sizeof(double) * c.nfij * (size_t)w.width;
         const long blocks_w = (long)k.npairs_ij * w.n_win;
-        if (bytes + c.lds_static[1] <= lim.lds_block && blocks_w <= INT_MAX &&
+        if (bytes + c.lds_static[1] <= lim.lds_block &&
             (a.kl_win_policy == 1 || blocks_w >= TEAM_KWIN_MIN_ITEMS)) {
             it.d.pairs_kl = w.pairs; it.d.q_kl = w.q; it.d.pdata_kl = w.pdata; it.d.win = w.win;
             it.d.use_lds = 2 | KR_WIN;
@@ -242,6 +242,36 @@ struct Launch {
     double cost;
 };
 
+// Workgroups of one launch: a grid holds fewer than 2^32 threads (the dispatch
+// packet counts them in 32 bits), and the kernels count workgroups in an int.
+static long max_blocks(int threads)
+{
+    return std::min((long)INT_MAX, (long)UINT32_MAX / threads);
+}
+
+// Appends an item; one above the limit of a launch in runs of its ij pairs.
+// false when the workgroups of one ij pair exceed it.
+static bool add_item(std::vector<Item> &items, const Item &it, int threads)
+{
+    const int npairs = it.d.npairs_ij;
+    const long most = max_blocks(threads), per_pair = it.blocks / npairs;
+    if (per_pair > most) return false;
+    const int step = (int)std::min((long)npairs, most / per_pair);
+    const int nij = (it.d.prims_ij & 0xffff) * (it.d.prims_ij >> 16);
+    for (long p0 = 0; p0 < npairs; p0 += step) {
+        Item part = it;
+        TaskDesc &d = part.d;
+        d.npairs_ij = (int)std::min((long)step, npairs - p0);
+        d.pairs_ij += p0;
+        d.q_ij += p0;
+        d.pdata_ij += p0 * nij * PREC;
+        part.blocks = per_pair * d.npairs_ij;
+        part.cost = it.cost * d.npairs_ij / npairs;
+        items.push_back(part);
+    }
+    return true;
+}
+
 // Cuts the items of one kernel into launches.  Items with the same LDS need go
 // together; others only join when the whole class leaves CUs idle anyway,
 // so that no item is held to the workgroups per CU of a wider one.
@@ -264,7 +294,7 @@ static void make_launches(std::vector<Item> &items, const Kernel &kernel, int cu
     int last_cu = 0;
     for (const Item &it : items) {
         if (last_cu == 0 || out.back().b.n == JK_BATCH || (!merge && it.per_cu != last_cu) ||
-            out.back().blocks + it.blocks > INT_MAX) {
+            out.back().blocks + it.blocks > max_blocks(kernel.threads)) {
             out.push_back(Launch());
             Launch &l = out.back();
             l.k = kernel;
@@ -284,8 +314,8 @@ static void make_launches(std::vector<Item> &items, const Kernel &kernel, int cu
     }
 }
 
-hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
-                           void *const *streams, int nstreams, const JKRun &run)
+static hipError_t plan_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                             const JKRun &run, std::vector<Launch> &launches)
 {
     const DeviceLimits lim = device_limits();
     const int pm = a.fp32_cut > -1e29f ? 0 : 1;
@@ -295,14 +325,12 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
     std::map<int, Group> by_kernel;
     std::vector<int> order;
     auto add = [&](int key, const Kernel &kern, const Item &it) {
-        if (it.blocks > INT_MAX) return false;
         Group &g = by_kernel[3 * key + kern.part];
         if (g.items.empty()) {
             order.push_back(3 * key + kern.part);
             g.k = kern;
         }
-        g.items.push_back(it);
-        return true;
+        return add_item(g.items, it, kern.threads);
     };
     for (int t = ntasks - 1; t >= 0; --t) {
         const JKTask &k = tasks[t];
@@ -372,9 +400,38 @@ hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks
             if (!add(key, kern, it)) return hipErrorInvalidConfiguration;
         }
     }
-    std::vector<Launch> launches;
     for (int key : order)
         make_launches(by_kernel[key].items, by_kernel[key].k, lim.cus, launches);
+    return hipSuccess;
+}
+
+hipError_t jk_plan_launches(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                            const JKRun &run, JKPlanItem *out, int nmax, int &n)
+{
+    std::vector<Launch> launches;
+    const hipError_t err = plan_tasks(a, tasks, ntasks, run, launches);
+    if (err != hipSuccess) return err;
+    n = 0;
+    for (size_t l = 0; l < launches.size(); ++l) {
+        const Launch &la = launches[l];
+        for (int i = 0; i < la.b.n; ++i, ++n) {
+            if (n >= nmax) continue;
+            const TaskDesc &d = la.b.t[i];
+            const long end = i + 1 < la.b.n ? la.b.block0[i + 1] : la.blocks;
+            out[n] = JKPlanItem{(int)l, la.k.threads, la.k.part, d.counter,
+                                (int)(d.pairs_ij - tasks[d.counter].pairs_ij), d.npairs_ij,
+                                la.b.block0[i], end - la.b.block0[i]};
+        }
+    }
+    return hipSuccess;
+}
+
+hipError_t jk_launch_tasks(const JKBuildArgs &a, const JKTask *tasks, int ntasks,
+                           void *const *streams, int nstreams, const JKRun &run)
+{
+    std::vector<Launch> launches;
+    const hipError_t planned = plan_tasks(a, tasks, ntasks, run, launches);
+    if (planned != hipSuccess) return planned;
     // each launch on the stream with the least work so far, in class order
     // (sorted by the estimate: 54 -> 60 ms on the 8-water two-density build;
     // round-robin: the 16-water range-separated K 144 -> 148 ms)

@@ -117,7 +117,14 @@ class JKTask(ctypes.Structure):
         ('kl_win', JKWindows * 2), ('swap_ijkl', ctypes.c_int)]
 
 
-EXPORTS = ('jk_build', 'jk_build_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
+class JKPlanItem(ctypes.Structure):
+    '''JKPlanItem of include/jkhip.h: a task's share of a planned launch.'''
+    _fields_ = [(n, ctypes.c_int) for n in ('launch', 'threads', 'part', 'task', 'pair0',
+                                            'npairs')] + [
+        ('block0', ctypes.c_int64), ('blocks', ctypes.c_int64)]
+
+
+EXPORTS = ('jk_build', 'jk_build_tasks', 'jk_plan_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
            'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_energy_ip1_tasks', 'jk_md_dm_to_hermite', 'jk_md_hermite_to_j',
            'jk_md_build_j', 'jk_int1e', 'jk_ao_transform', 'mlp_gemm_bf16', 'mlp_silu_backward', 'mlp_colsum', 'mlp_mse_grad',
            'mlp_adamw', 'mlp_to_bf16', 'jk_last_error', 'jk_abi_version')
@@ -135,7 +142,7 @@ def load():
                            'or make -C gpu4pyscf_amd/csrc')
     lib = ctypes.CDLL(LIB_PATH)
     lib.jk_last_error.restype = ctypes.c_char_p
-    for name in ('jk_build', 'jk_build_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
+    for name in ('jk_build', 'jk_build_tasks', 'jk_plan_tasks', 'jk_pair_data', 'jk_ovlp_mask', 'jk_pair_qcond', 'jk_dm_cond',
                  'jk_dm_cond_noalloc', 'jk_energy_ip1', 'jk_energy_ip1_tasks', 'jk_abi_version'):
         getattr(lib, name).restype = ctypes.c_int
     lib.jk_build.argtypes = [ctypes.POINTER(JKBuildArgs), c_void_p]

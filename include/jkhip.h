@@ -214,6 +214,24 @@ int jk_energy_ip1_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks
                         int n_copies, int64_t copy_stride, double j_factor, double k_factor,
                         void *const *streams, int nstreams);
 
+/* One task, or a run of its ij pairs, in a launch of a plan. */
+typedef struct {
+    int launch;                     /* launches are numbered in their order */
+    int threads;                    /* per workgroup */
+    int part;                       /* 0; 1 and 2: the two parts of an operator */
+    int task;
+    int pair0, npairs;              /* ij pairs [pair0, pair0 + npairs) of the task */
+    int64_t block0, blocks;         /* workgroups of the item within its launch */
+} JKPlanItem;
+
+/* The launches of jk_build_tasks (gradient == 0) or jk_energy_ip1_tasks
+ * (gradient != 0; j_factor = k_factor = 1) for these arguments, without any of
+ * them: *nitems is set to the number of items, the first nmax of which are
+ * written to out.  Reads no device memory and runs without a GPU, with the
+ * occupancies of one workgroup per CU then. */
+int jk_plan_tasks(const JKBuildArgs *args, const JKTask *tasks, int ntasks, int gradient,
+                  JKPlanItem *out, int nmax, int *nitems);
+
 /* ---- McMurchie-Davidson J-engine (basis of single-primitive shells,
  * SortedGTO(decontract=True)).  Replaces the reference's MD J path
  * (gpu4pyscf/scf/j_engine.py:50-236; dm_to_Rt / MD_build_j / Rt_to_dm of
