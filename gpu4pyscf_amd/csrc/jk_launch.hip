@@ -181,11 +181,17 @@ static int plan_lane(const JKBuildArgs &a, const JKTask &k, const ClassInfo &c, 
     // Two densities, ms, any-number kernel -> this: 8 waters def2-SVP 6.6 -> 3.4,
     // 8 and 12 waters def2-TZVP 53.6 -> 36.1 and 143 -> 75; 12 waters in two
     // launches of one density 92.
+    // J only of more than two densities: s and p classes stay on the any-number
+    // kernel, whose J costs less than evaluating their integrals again for each two
+    // (eight densities, ms, in pairs -> together: 64 waters STO-3G 117 -> 95 on one
+    // stream, all s and p; 32 waters def2-SVP (ps|ss) 36.2 -> 30.1, (ss|ss) 21.0 ->
+    // 17.1, but (dp|ps) 8.7 -> 14.6, (dp|ds) 2.3 -> 5.6, (dp|ss) 3.9 -> 6.0).
+    const bool together = !a.vk && a.n_dm > 2 && k.li <= 1;
     Item one = it;
-    const bool fast = pm == 1 && (a.n_dm == 1 ||
-                                  (a.n_dm <= FAST_DM_MAX && c.fn[JK_FAST + what] &&
-                                   plan_lane_rows(a, k, c, JK_FAST + what, lim, one) &&
-                                   (a.n_dm == 2 || one.blocks > lim.cus)));
+    const bool fast = pm == 1 && !together &&
+                      (a.n_dm == 1 || (a.n_dm <= FAST_DM_MAX && c.fn[JK_FAST + what] &&
+                                       plan_lane_rows(a, k, c, JK_FAST + what, lim, one) &&
+                                       (a.n_dm == 2 || one.blocks > lim.cus)));
     const bool two = fast && n_dm >= 2;
     const bool four = fast && a.vk && k.npairs_kl >= FOUR_MIN_KL;
     // in order of preference

@@ -129,3 +129,15 @@ def test_plan_of_nothing_and_bad_arguments():
     assert lib.jk_plan_tasks(ctypes.byref(a), tasks, 1, 0, None, 3, ctypes.byref(n)) == 1
     _task(tasks[0], (clib.JK_LMAX + 1, 0, 0, 0), 3, 3)
     assert lib.jk_plan_tasks(ctypes.byref(a), tasks, 1, 0, None, 0, ctypes.byref(n)) == 2
+
+
+# J of many densities: classes of s and p shells digest all of them beside one
+# evaluation of the integrals, the others in pairs
+@pytest.mark.parametrize('ls,vk,times', [((0, 0, 0, 0), False, 1), ((1, 1, 1, 0), False, 1),
+                                         ((2, 0, 1, 0), False, 3), ((1, 1, 1, 0), True, 3)])
+def test_many_densities_evaluate_the_integrals_once_where_that_is_faster(ls, vk, times):
+    from gpu4pyscf_amd.lib import clib
+    tasks = (clib.JKTask * 1)()
+    _task(tasks[0], ls, 20000, 20000, nao=100)
+    _check(_args(n_dm=6, vk=vk), tasks, times=times)
+    _check(_args(n_dm=2, vk=vk), tasks)
