@@ -61,6 +61,8 @@ class _VHFOpt(jk_mod._VHFOpt):
         self.task_filter = lambda ls: sum(ls) > MD_LMAX
         self.last_md_quartets = None
         self.last_md_hash = None
+        # kl windows hold K rows, which a build of J has none of
+        self.kl_window_ao = self.kl_window_ao_team = 0
 
     def _make_sorted_mol(self):
         return SortedGTO(self.mol, decontract=True)
