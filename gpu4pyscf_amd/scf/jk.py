@@ -18,6 +18,7 @@ exists here).
 
 import contextlib
 import ctypes
+import functools
 import math
 import time
 
@@ -149,6 +150,13 @@ def class_kernel_name(ls):
     return f'{kind}<{ls[0]}, {ls[1]}, {ls[2]}, {ls[3]}>'
 
 
+@functools.lru_cache(maxsize=None)
+def has_lane_class(lk, ll):
+    '''Whether a per-lane class has a ket of angular momenta lk >= ll.'''
+    return any(class_kernel_name((li, lj, lk, ll)).startswith('jk_lane')
+               for li in range(lk, 4) for lj in range(li + 1))
+
+
 def _set_kl_win(a, sets):
     '''kl column windows of a JKTask / JKBuildArgs (sets: an entry of
     _VHFOpt._kl_windows, [per-lane, team], or None).'''
@@ -183,13 +191,21 @@ def kl_window_table(pairs, offs, ao_loc, nbas, k, l, W):
         spw = max(1, W // (nao // nsh))     # most shells per window
         spw = -(-nsh // -(-nsh // spw))     # the same number of windows, evened out
         return spw, -(-nsh // spw)
-    spk, _ = cut(k, k_nao)
+    spk, nwk = cut(k, k_nao)
     spl, nwl = cut(l, l_nao)
-    p = np.asarray(pairs).astype(np.int64)
-    ksh, lsh = p // nbas, p % nbas
-    key = ((ksh - offs[k]) // spk) * nwl + (lsh - offs[l]) // spl
+    # window of every pair, by tables over the shells; 16 bits where they hold it
+    # (numpy sorts those by radix)
+    p = np.asarray(pairs, dtype=np.uint32)
+    ksh = p // np.uint32(nbas)
+    lsh = p - ksh * np.uint32(nbas)
+    kind = np.int16 if nwk * nwl < 2**15 else np.int64
+    sh = np.arange(nbas, dtype=np.int64)
+    key = (((sh - offs[k]) // spk * nwl).astype(kind)[ksh] +
+           ((sh - offs[l]) // spl).astype(kind)[lsh])
     order = np.argsort(key, kind='stable')
-    ids, first = np.unique(key[order], return_index=True)
+    key = key[order]
+    first = np.flatnonzero(np.append(True, key[1:] != key[:-1]))
+    ids = key[first].astype(np.int64)
     end = np.append(first[1:], len(p))
     a, b = np.divmod(ids, nwl)
     k0 = offs[k] + a * spk
@@ -366,26 +382,35 @@ class _VHFOpt:
         '''kl column windows of every group pair wider than the window in k
         or in l: {(k, l): [lane windows, team windows]}, each None or
         (pairs, q, pdata, table, width), the device copies of
-        kl_window_table's reordering and window rows.'''
+        kl_window_table's reordering and window rows.  A ket that no per-lane class
+        has gets none, but the team windows of kl_win_policy 1.'''
         torch = _torch()
         mol = self.sorted_mol
-        out = {}
+        ls = mol.uniq_l_ctr[:, 0]
+        found = []          # (k, l), set, (order, table, width)
         for (k, l), (p, _, _) in cache.items():
-            sets = []
-            for W in (int(self.kl_window_ao), int(self.kl_window_ao_team)):
-                w = (kl_window_table(p, mol.group_offsets, mol.ao_loc, mol.nbas, k, l, W)
-                     if W > 0 else None)
-                if w is None:
-                    sets.append(None)
-                    continue
-                order, tab, width = w
-                dev = dev_pairs[k, l].device
-                o = torch.as_tensor(order, device=dev)
-                sets.append((dev_pairs[k, l][o].contiguous(), dev_q[k, l][o].contiguous(),
-                             dev_pd[k, l][o].contiguous(), torch.as_tensor(tab, device=dev),
-                             width))
-            if sets[0] is not None or sets[1] is not None:
-                out[k, l] = sets
+            lane = has_lane_class(int(ls[k]), int(ls[l]))
+            for n, W in enumerate((self.kl_window_ao, self.kl_window_ao_team)):
+                if W > 0 and (lane or n == 1 and self.kl_win_policy == 1):
+                    w = kl_window_table(p, mol.group_offsets, mol.ao_loc, mol.nbas, k, l, int(W))
+                    if w is not None:
+                        found.append(((k, l), n, w))
+        out = {}
+        if not found:
+            return out
+        # one copy to the device for all orders, one for all tables (a pair of
+        # synchronous copies per set took longer than the gathers)
+        dev = next(iter(dev_pairs.values())).device
+        orders = torch.as_tensor(np.concatenate([w[0] for _, _, w in found]), device=dev)
+        tables = torch.as_tensor(np.concatenate([w[1] for _, _, w in found]), device=dev)
+        o0 = t0 = 0
+        for key, n, (order, tab, width) in found:
+            o, t = orders[o0:o0 + len(order)], tables[t0:t0 + len(tab)]
+            o0 += len(order)
+            t0 += len(tab)
+            out.setdefault(key, [None, None])[n] = (
+                dev_pairs[key].index_select(0, o), dev_q[key].index_select(0, o),
+                dev_pd[key].index_select(0, o), t, width)
         return out
 
     def _order_pairs(self, q, split):
