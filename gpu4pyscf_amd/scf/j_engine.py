@@ -190,6 +190,9 @@ class _VHFOpt(jk_mod._VHFOpt):
                     ptr(vj[n]), ptr(jh[key]), nao, ptr(pairs), len(pairs),
                     ptr(d['pdata'][key]), li, lj, ptr(d['bas']), ptr(d['env']),
                     ptr(d['ao_loc']), nbas, stream), 'jk_md_hermite_to_j')
+        if vj_rys is None and self.tasks():
+            # (no density: refused there)
+            vj_rys = super().get_jk(dms, 1, with_k=False, screen='j')[0]
         if vj_rys is not None:
             vj += vj_rys
         if counter is not None:
