@@ -30,10 +30,11 @@ from gpu4pyscf_amd.lib import clib
 __all__ = ['get_jk', 'get_j', 'get_k', '_VHFOpt']
 
 TILE = 12                 # pair enumeration tile, gpu4pyscf/scf/jk.py:51
-# widest kl column windows (AOs of k, and of l) for the LDS K rows of the per-lane
-# kernels: bra blocks below 9 AOs, and larger ones
+# widest kl column windows (AOs of k, and of l) for the LDS K rows: of the per-lane
+# kernels with bra blocks below 9 AOs; of those with larger ones, and of the team
+# kernels under kl_win_policy 1
 KL_WINDOW_AO = 256
-KL_WINDOW_AO_NARROW = 128
+KL_WINDOW_AO_TEAM = 128
 Q_COND_MARGIN = 4.        # bin width of the descending q_cond ordering
 LMAX = clib.JK_LMAX
 
@@ -254,7 +255,7 @@ class _VHFOpt:
         # block on the bra side (JKBuildArgs.swap_ijkl)
         self.swap_tasks = True
         self.kl_window_ao = KL_WINDOW_AO
-        self.kl_window_ao_team = KL_WINDOW_AO_NARROW
+        self.kl_window_ao_team = KL_WINDOW_AO_TEAM
         self.kl_win_policy = 0
 
     def profile_results(self):

@@ -71,3 +71,11 @@ def test_launches_of_other_kets_use_no_windows():
                                       for n_dm in (1, 2) for vj, vk in ((1, 1), (1, 0), (0, 1))
                                       for fp32 in (False, True)])
                     assert plans[0] == plans[1]
+
+
+def test_window_defaults_by_name():
+    from gpu4pyscf_amd.gto.mole import M
+    from gpu4pyscf_amd.scf import jk
+    opt = jk._VHFOpt(M(atom='H 0 0 0; H 0 0 1', basis='sto-3g'))
+    assert opt.kl_window_ao == jk.KL_WINDOW_AO
+    assert opt.kl_window_ao_team == jk.KL_WINDOW_AO_TEAM
