@@ -133,11 +133,6 @@
 #ifndef LANE_DROWS
 #define LANE_DROWS      1
 #endif
-// rank the per-lane LDS row candidates by the workgroups per CU their LDS
-// allows (0: take the largest rows that fit)
-#ifndef LANE_KROWS_OCC
-#define LANE_KROWS_OCC  1
-#endif
 // K_ik / K_jk LDS rows of the per-lane kernel: 1 = the lanes of a run of
 // equal k shell first sum their values across the wavefront and the run's
 // last lane adds once (no same-address LDS atomics within the run), 0 = every
