@@ -233,7 +233,7 @@ def main():
             ps = tuple(int(uniq[x, 1]) for x in t)
             f = cnt * quartet_flops(ls, ps, 1)
             total += f
-            a = by.setdefault(jk.class_kernel_name(ls), [0., 0., 0, 0])
+            a = by.setdefault(jk.class_kernel_name(ls, 1), [0., 0., 0, 0])
             a[0] += ms; a[1] += f; a[2] += nl; a[3] += cnt
         return by, total
 
@@ -256,7 +256,8 @@ def main():
         v = by_serial[key]
         log(f'    {key}: {v[0]:8.2f} ms  {tflops(v[1], v[0]):.2f} TFLOP/s  '
             f'avg launch {v[0] / v[2] * 1e3:.1f} us  launches {v[2]}  quartets {v[3]}')
-    for kind in ('jk_lane_kernel', 'jk_team_kernel', 'jk_generic_kernel'):
+    for kind in ('jk_lane_fast_kernel', 'jk_lane_kernel', 'jk_team_kernel',
+                 'jk_generic_kernel'):
         sel = [v for k, v in by_serial.items() if k.startswith(kind)]
         if sel:
             ms, fl = sum(v[0] for v in sel), sum(v[1] for v in sel)

@@ -116,7 +116,7 @@ def group_by_split_points(q, split_points):
     return np.concatenate(subsets).astype(np.int64)
 
 
-LANE_MAX = 170      # LANE_MAX of csrc/jk_kernels.hip
+LANE_MAX = 170      # LANE_MAX of csrc/jk_class_kernels.h
 # class launches run on this many streams (32-water def2-TZVP build, ms:
 # 1 -> 648, 2 -> 569, 3 -> 564, 4 -> 566 with four-wave per-lane blocks;
 # 2 -> 482, 3 -> 463, 4 -> 454 with two-wave blocks).  HIP gives a process
@@ -135,12 +135,14 @@ LANE_CHUNKED = {(3, 1, 2, 0), (3, 2, 1, 0), (2, 1, 1, 1), (2, 2, 2, 0), (3, 1, 1
                 (3, 3, 1, 0), (3, 1, 3, 0)}
 
 
-def class_kernel_name(ls):
+def class_kernel_name(ls, n_dm=None):
     '''Name of the HIP kernel template that evaluates angular class ls =
     (li, lj, lk, ll): the per-lane kernel when the Cartesian block and the
     three 2D tables fit in LANE_MAX doubles or the class is one of
     LANE_CHUNKED, else the team kernel; classes with a shell of l >= 4 run
-    on the runtime-l kernel.'''
+    on the runtime-l kernel.  With n_dm, the template of an FP64 build of J
+    and K of that many densities (1 or 2) whose rows fit in LDS: all per-lane
+    classes but the chunked ones with an f shell on jk_lane_fast_kernel.'''
     if max(ls) > 3:
         return f'jk_generic_kernel<{ls[0]}, {ls[1]}, {ls[2]}, {ls[3]}>'
     nc = [(l + 1) * (l + 2) // 2 for l in ls]
@@ -148,6 +150,8 @@ def class_kernel_name(ls):
     gs = (ls[0] + 1) * (ls[1] + 1) * (ls[2] + 1) * (ls[3] + 1)
     lane = nf + 3 * gs <= LANE_MAX or tuple(ls) in LANE_CHUNKED
     kind = 'jk_lane_kernel' if lane else 'jk_team_kernel'
+    if lane and n_dm in (1, 2) and not (ls[0] == 3 and tuple(ls) in LANE_CHUNKED):
+        kind = 'jk_lane_fast_kernel'
     return f'{kind}<{ls[0]}, {ls[1]}, {ls[2]}, {ls[3]}>'
 
 

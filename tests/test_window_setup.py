@@ -79,3 +79,14 @@ def test_window_defaults_by_name():
     opt = jk._VHFOpt(M(atom='H 0 0 0; H 0 0 1', basis='sto-3g'))
     assert opt.kl_window_ao == jk.KL_WINDOW_AO
     assert opt.kl_window_ao_team == jk.KL_WINDOW_AO_TEAM
+
+
+def test_kernel_names_of_fp64_builds():
+    from gpu4pyscf_amd.scf import jk
+    for ls, name in (((1, 0, 1, 0), 'jk_lane_fast_kernel'), ((2, 1, 1, 1), 'jk_lane_fast_kernel'),
+                     ((3, 1, 2, 0), 'jk_lane_kernel'), ((3, 0, 2, 1), 'jk_team_kernel'),
+                     ((4, 0, 0, 0), 'jk_generic_kernel')):
+        args = ', '.join(map(str, ls))
+        assert jk.class_kernel_name(ls, 1) == jk.class_kernel_name(ls, 2) == f'{name}<{args}>'
+        assert jk.class_kernel_name(ls) == f"{name.replace('fast_', '')}<{args}>"
+        assert jk.class_kernel_name(ls, 3) == jk.class_kernel_name(ls)
