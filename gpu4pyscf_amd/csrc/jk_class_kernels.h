@@ -1,6 +1,6 @@
-// Device code of the class kernels (per-lane and team kernels) and their
-// host launchers, shared by the translation units that instantiate the
-// angular classes (jk_classes.hip, compiled once per part).
+// Device code of the class kernels (per-lane and team kernels) and the class
+// information for their launches (jk_launch.hip), shared by the translation units
+// that instantiate the angular classes (jk_classes.hip, compiled once per part).
 // Direct-SCF J/K kernels for MI355X (gfx950), FP64 Rys quadrature.
 //
 // One launch evaluates one angular class (li,lj,lk,ll) of screened shell

@@ -10,7 +10,7 @@
 // shells have few of them, so the items are cut small: with one wavefront per
 // 256 candidates and the whole block per wavefront, one water molecule
 // (def2-TZVP with a g shell on each atom) ran 3-12 wavefronts per launch, up to
-// 146 ms for the (gg|gg) class, 357 ms per build; 10.2 ms now.
+// 146 ms for the (gg|gg) class, 357 ms per build; 9.2 ms now.
 // The first wavefront applies the survival predicate to the chunk; every
 // queued quartet is then evaluated by the whole workgroup, a batch of
 // (primitive quartet, root) combinations at a time:

@@ -3,8 +3,8 @@
 Drop-in for ``_jk_energy_per_atom`` (gpu4pyscf/grad/rhf.py:60-171): the first
 derivatives, per atom, of the two-electron energy of one (closed shell) or
 two (alpha, beta) densities, j_factor E_J - k_factor E_K, from the ERI
-first derivatives evaluated by the runtime-l Rys kernel of libjkhip.so
-(``jk_energy_ip1``).  The screening object is the J/K engine's ``_VHFOpt``;
+first derivatives evaluated by libjkhip.so (``jk_energy_ip1_tasks``): one quartet
+per lane for the small classes, the runtime-l Rys kernel for the others.  The screening object is the J/K engine's ``_VHFOpt``;
 the two-particle density and the survival predicate follow
 gpu4pyscf/lib/gvhf-rys/rys_contract_jk_ip1.cu:523-577,1789-1797 and
 create_tasks.cu:829-889.  Range separation follows the molecule's omega

@@ -241,8 +241,9 @@ class _VHFOpt:
         self.profile = False
         self._profile_pending = []
         # class tasks only add into vj/vk with atomics, so they may run
-        # concurrently: they are spread round-robin over nstreams streams
-        # (default priority) that join the caller's stream at the end
+        # concurrently: their launches go over nstreams streams (default
+        # priority), each on the one with the least work so far (round-robin
+        # with time_classes or profile), that join the caller's stream at the end
         self.nstreams = NSTREAMS
         self._streams = {}
         # copies of vj/vk the class kernels add into (one per XCD)

@@ -35,7 +35,7 @@ extern "C" {
  * Moment rows (rules of n = 1, 2, 3 roots): 79, 95 and 109 rows (boys_rows in
  * all) of JK_BOYS_M doubles each, the rows of n after those of n - 1, from
  * coef[boys] on, 16-byte aligned; row g holds F_{2n-1+k}(x_g) / k! for k < 12, exp(-x_g) and 0 for
- * x_g = g * boys_step (0.5), covering x < xmax[n-1]. */
+ * x_g = g * boys_step (0.5), covering x < xmax[n-1]; boys_inv_step is not read. */
 #define JK_BOYS_M       14
 typedef struct {
     const double *coef;
