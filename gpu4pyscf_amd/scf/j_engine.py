@@ -16,6 +16,7 @@ reference's J-engine: tile 1, bin 0 dropped, sorted by descending q_cond
 (j_engine.py:239-259).
 '''
 
+import contextlib
 import ctypes
 import math
 import os
@@ -30,6 +31,7 @@ __all__ = ['get_j', '_VHFOpt']
 
 MD_LMAX = 4           # li + lj + lk + ll of the Hermite kernels
 MD_PAIR_LMAX = 4      # largest l of a shell in the Hermite transforms
+MD_FORK_WORK = 1e6    # estimated work of a density from which side streams pay
 BOYS_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                          'csrc', 'md_boys_table.npz')
 
@@ -91,7 +93,22 @@ class _VHFOpt(jk_mod._VHFOpt):
         # every bra group pair against every ket group pair within MD_LMAX
         self._md_tasks = [(a, b) for a in keys for b in keys
                           if sum(self._md_l[a]) + sum(self._md_l[b]) <= MD_LMAX]
+        # rough work of each task, and its stream by the number of streams
+        self._md_work = [float(len(d['pairs'][a])) * len(d['pairs'][b]) *
+                         (_nh(sum(self._md_l[a])) * _nh(sum(self._md_l[b])) + 60)
+                         for a, b in self._md_tasks]
+        self._md_lanes = {}
         return self
+
+    def _lanes(self, n):
+        '''Stream of each Hermite task, of n: the one with the least work so far.'''
+        if n not in self._md_lanes:
+            load, out = [0.] * n, []
+            for w in self._md_work:
+                out.append(load.index(min(load)))
+                load[out[-1]] += w
+            self._md_lanes[n] = out
+        return self._md_lanes[n]
 
     def md_tasks(self):
         return list(self._md_tasks)
@@ -124,6 +141,9 @@ class _VHFOpt(jk_mod._VHFOpt):
         dm_cond = torch.empty((nbas, nbas), dtype=torch.float32, device=dev)
         work = torch.empty((nbas, nbas), dtype=torch.float64, device=dev)
         vj_rys = None
+        # classes above MD_LMAX: Rys J-only build on the same pair lists
+        rys = bool(self.tasks())
+        fork = sum(self._md_work) >= MD_FORK_WORK
         for n in range(dms.shape[0]):
             dm = dms[n]
             clib.check(lib.jk_dm_cond(ptr(dm_cond), ptr(work), ptr(dm), 1, nao,
@@ -156,14 +176,17 @@ class _VHFOpt(jk_mod._VHFOpt):
             args.dm_penalty = dm_penalty
             # the molecule's operator (screening q_cond uses the same)
             args.omega = float(getattr(self.mol, 'omega', 0.) or 0.)
-            # the tasks over the side streams, each on the one with the least work
-            # so far; the Rys build beside the last density's reads a maximum of
-            # its own on the caller's stream before it launches, and must not wait
-            # for them (16 waters def2-TZVP: 47.9 ms one after the other)
-            with self.fork_streams(dev) as streams:
-                side = streams[1:] or streams
-                load = [0.] * len(side)
-                for a, b in self._md_tasks:
+            # the tasks over the side streams, unless they are too small for the
+            # 0.1 ms that takes (H2 STO-3G 0.12 -> 0.22 ms, 1 water 0.28 -> 0.38;
+            # 2 waters 0.80 -> 0.57); the Rys build beside the last density's
+            # reads a maximum of its own on the caller's stream before it launches,
+            # and must not wait for them (16 waters def2-TZVP: 47.9 ms one after
+            # the other)
+            last = rys and n == dms.shape[0] - 1
+            with (self.fork_streams(dev) if last or fork else
+                  contextlib.nullcontext([])) as streams:
+                side = [ctypes.c_void_p(s.cuda_stream) for s in streams[1:]] or [stream]
+                for (a, b), lane in zip(self._md_tasks, self._lanes(len(side))):
                     args.lij, args.lkl = sum(self._md_l[a]), sum(self._md_l[b])
                     args.npairs_ij, args.npairs_kl = len(d['pairs'][a]), len(d['pairs'][b])
                     args.pdata_ij = d['pdata'][a].data_ptr()
@@ -174,14 +197,9 @@ class _VHFOpt(jk_mod._VHFOpt):
                     args.pairs_kl = d['pairs'][b].data_ptr()
                     args.dh_kl = dh[b].data_ptr()
                     args.jh_ij = jh[a].data_ptr()
-                    s = load.index(min(load))
-                    load[s] += (float(args.npairs_ij) * args.npairs_kl *
-                                (_nh(args.lij) * _nh(args.lkl) + 60))
-                    clib.check(lib.jk_md_build_j(ctypes.byref(args),
-                                                 ctypes.c_void_p(side[s].cuda_stream)),
+                    clib.check(lib.jk_md_build_j(ctypes.byref(args), side[lane]),
                                'jk_md_build_j')
-                if n == dms.shape[0] - 1 and self.tasks():
-                    # classes above MD_LMAX: Rys J-only build on the same pair lists
+                if last:
                     vj_rys = super().get_jk(dms, 1, with_k=False, screen='j')[0]
             for key in self._md_keys:
                 li, lj = self._md_l[key]
@@ -190,8 +208,7 @@ class _VHFOpt(jk_mod._VHFOpt):
                     ptr(vj[n]), ptr(jh[key]), nao, ptr(pairs), len(pairs),
                     ptr(d['pdata'][key]), li, lj, ptr(d['bas']), ptr(d['env']),
                     ptr(d['ao_loc']), nbas, stream), 'jk_md_hermite_to_j')
-        if vj_rys is None and self.tasks():
-            # (no density: refused there)
+        if rys and vj_rys is None:      # no density: refused there
             vj_rys = super().get_jk(dms, 1, with_k=False, screen='j')[0]
         if vj_rys is not None:
             vj += vj_rys
